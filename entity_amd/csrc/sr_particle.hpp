@@ -150,15 +150,32 @@ __device__ __forceinline__ float lin3(const A& F, int c, int ia, int ja, int ka,
 }
 
 // ---- interpolation, B-spline orders: sr.hpp:1170-1366 ------------------------
+// Through GlobalEMAhead a component's stencil values are all loaded before the
+// first is used, so that they are one round trip to memory; left to itself the
+// compiler uses each row as it arrives to save registers, and a 3D order-2
+// gather is then some 18 round trips.  The arithmetic is the same.
+struct GlobalEMAhead : GlobalEM {};
+template <class A> struct LoadsAhead { static constexpr bool value = false; };
+template <> struct LoadsAhead<GlobalEMAhead> { static constexpr bool value = true; };
+
 template <int O, class A>
 __device__ __forceinline__ float spl2(const A& F, int c, int imin, int jmin, const float* S1,
                                       const float* S2) {
+  float v[O + 1][O + 1];
+  if constexpr (LoadsAhead<A>::value) {
+#pragma unroll
+    for (int b = 0; b < O + 1; b++)
+#pragma unroll
+      for (int a = 0; a < O + 1; a++) v[b][a] = F(c, imin + a, jmin + b, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   float e = ZERO;
 #pragma unroll
   for (int b = 0; b < O + 1; b++) {
     float c0 = ZERO;
 #pragma unroll
-    for (int a = 0; a < O + 1; a++) c0 += S1[a] * F(c, imin + a, jmin + b, 0);
+    for (int a = 0; a < O + 1; a++)
+      c0 += S1[a] * (LoadsAhead<A>::value ? v[b][a] : F(c, imin + a, jmin + b, 0));
     e += c0 * S2[b];
   }
   return e;
@@ -167,6 +184,16 @@ __device__ __forceinline__ float spl2(const A& F, int c, int imin, int jmin, con
 template <int O, class A>
 __device__ __forceinline__ float spl3(const A& F, int c, int imin, int jmin, int kmin,
                                       const float* S1, const float* S2, const float* S3) {
+  float v[O + 1][O + 1][O + 1];
+  if constexpr (LoadsAhead<A>::value) {
+#pragma unroll
+    for (int g = 0; g < O + 1; g++)
+#pragma unroll
+      for (int b = 0; b < O + 1; b++)
+#pragma unroll
+        for (int a = 0; a < O + 1; a++) v[g][b][a] = F(c, imin + a, jmin + b, kmin + g);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   float e = ZERO;
 #pragma unroll
   for (int g = 0; g < O + 1; g++) {
@@ -175,7 +202,9 @@ __device__ __forceinline__ float spl3(const A& F, int c, int imin, int jmin, int
     for (int b = 0; b < O + 1; b++) {
       float c00 = ZERO;
 #pragma unroll
-      for (int a = 0; a < O + 1; a++) c00 += S1[a] * F(c, imin + a, jmin + b, kmin + g);
+      for (int a = 0; a < O + 1; a++)
+        c00 += S1[a] *
+               (LoadsAhead<A>::value ? v[g][b][a] : F(c, imin + a, jmin + b, kmin + g));
       c0 += c00 * S2[b];
     }
     e += c0 * S3[g];

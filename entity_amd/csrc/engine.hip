@@ -17,7 +17,11 @@ namespace {
 struct Profile {
   std::mutex                                  mu;
   bool                                        on = false;
-  std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
+  struct Pending {
+    std::pair<hipEvent_t, hipEvent_t> ev;
+    int                               species;  // pushed between the two events
+  };
+  std::vector<Pending>                        pending;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> spare;
   double                                      ms = 0.0;
   int64_t                                     launches = 0;
@@ -41,9 +45,9 @@ bool prof_begin(hipStream_t st, std::pair<hipEvent_t, hipEvent_t>* ev) {
   return true;
 }
 
-void prof_end(hipStream_t st, const std::pair<hipEvent_t, hipEvent_t>& ev) {
+void prof_end(hipStream_t st, const std::pair<hipEvent_t, hipEvent_t>& ev, int species) {
   std::lock_guard<std::mutex> lk(g_prof.mu);
-  if (hipEventRecord(ev.second, st) == hipSuccess) g_prof.pending.push_back(ev);
+  if (hipEventRecord(ev.second, st) == hipSuccess) g_prof.pending.push_back({ ev, species });
 }
 
 bool same_grid(const FieldView& a, const FieldView& b) {
@@ -261,21 +265,25 @@ ntt_status sr_step(ntt_field_t* em, ntt_field_t* cur, ntt_field_t* buff, ntt_spe
   // currents.h:68: J = 0 -- here the fixed-point accumulator (a fill kernel
   // rather than a memset, so that the step can be captured in a graph)
   if (prm->deposit_enable) launch_zero_u64(P.acc, J.cstride * 3, st);
-  for (int sp = 0; sp < nspecies; ++sp) {
-    const Prep& p = P.prep[sp];
-    if (!p.run) continue;
-    const int ppt = prm->particles_per_thread > 0 ? prm->particles_per_thread : 4;
+  {
+    std::vector<SpeciesPush> push;
+    push.reserve(nspecies);
+    for (int sp = 0; sp < nspecies; ++sp) {
+      const Prep& p = P.prep[sp];
+      if (!p.run) continue;
+      void* recs = (P.recs != nullptr && P.rec_stride > 0)
+                     ? static_cast<char*>(P.recs) + P.rec_stride * static_cast<uint64_t>(sp)
+                     : P.recs;
+      push.push_back({ p.pv, p.ndth, species[sp].charge, p.dep, p.alg, species[sp].tile_offsets,
+                       species[sp].ntiles, recs });
+    }
     std::pair<hipEvent_t, hipEvent_t> ev;
-    const bool timed = timed_ok && prof_begin(st, &ev);
-    void* recs = (P.recs != nullptr && P.rec_stride > 0)
-                   ? static_cast<char*>(P.recs) + P.rec_stride * static_cast<uint64_t>(sp)
-                   : P.recs;
-    s = launch_push_deposit_periodic(p.pv, E, J, P.acc, P.D, prm->shape_order, p.alg, p.ndth,
-                                     P.dt, metric->dx, species[sp].charge, p.dep, P.fscale,
-                                     species[sp].tile_offsets, species[sp].ntiles, ppt,
-                                     P.flags, P.flag_chunks, recs, P.rec_chunks,
-                                     P.rec_stride > 0, st);
-    if (timed) prof_end(st, ev);
+    const bool timed = timed_ok && !push.empty() && prof_begin(st, &ev);
+    s = launch_push_deposit_periodic(push.data(), static_cast<int>(push.size()), E, J, P.acc, P.D,
+                                     prm->shape_order, P.dt, metric->dx, P.fscale,
+                                     prm->particles_per_thread > 0 ? prm->particles_per_thread : 4,
+                                     P.flags, P.flag_chunks, P.rec_chunks, P.rec_stride > 0, st);
+    if (timed) prof_end(st, ev, static_cast<int>(push.size()));
     if (s != NTT_OK) return s;
   }
   if (prm->deposit_enable) {
@@ -656,13 +664,13 @@ extern "C" ntt_status ntt_profile_enable(int32_t on) {
 
 extern "C" ntt_status ntt_profile_read(double* ms_total, int64_t* launches, int32_t reset) {
   std::lock_guard<std::mutex> lk(g_prof.mu);
-  for (auto& ev : g_prof.pending) {
-    if (hipEventSynchronize(ev.second) != hipSuccess) return NTT_ERR_HIP;
+  for (auto& p : g_prof.pending) {
+    if (hipEventSynchronize(p.ev.second) != hipSuccess) return NTT_ERR_HIP;
     float ms = 0.0f;
-    if (hipEventElapsedTime(&ms, ev.first, ev.second) != hipSuccess) return NTT_ERR_HIP;
+    if (hipEventElapsedTime(&ms, p.ev.first, p.ev.second) != hipSuccess) return NTT_ERR_HIP;
     g_prof.ms += ms;
-    g_prof.launches += 1;
-    g_prof.spare.push_back(ev);
+    g_prof.launches += p.species;
+    g_prof.spare.push_back(p.ev);
   }
   g_prof.pending.clear();
   if (ms_total) *ms_total = g_prof.ms;

@@ -16,14 +16,20 @@ ntt_status launch_deposit(const ParticleView& pv, const FieldView& J, int D, int
                           float charge, float dt, hipStream_t st);
 
 // push_deposit.hip
-ntt_status launch_push_deposit_periodic(const ParticleView& pv, const FieldView& em,
-                                        const FieldView& cur, unsigned long long* acc,
-                                        int D, int order, int alg,
-                                        float ndth, float dt, float dxm, float charge,
-                                        bool deposit, float fscale,
-                                        const uint32_t* tile_offsets,
-                                        int64_t ntiles, int ppt, uint32_t* flags,
-                                        int64_t flag_chunks, void* recs, int64_t rec_chunks,
+// one species' part of a step's push and deposit
+struct SpeciesPush {
+  ParticleView    pv;
+  float           ndth, charge;
+  bool            deposit;
+  int             alg;
+  const uint32_t* tile_offsets;
+  int64_t         ntiles;
+  void*           recs;  // split-path box records (null: none)
+};
+ntt_status launch_push_deposit_periodic(const SpeciesPush* sp, int nspecies, const FieldView& em,
+                                        const FieldView& cur, unsigned long long* acc, int D,
+                                        int order, float dt, float dxm, float fscale, int ppt,
+                                        uint32_t* flags, int64_t flag_chunks, int64_t rec_chunks,
                                         bool reuse_boxes, hipStream_t st);
 // bytes of the chunk flags of the split (push, then deposit) launches for up
 // to max_chunks chunks; `flags` above holds flag_chunks of them (null: the

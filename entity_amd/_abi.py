@@ -210,6 +210,9 @@ SIGNATURES: dict[str, tuple] = {
                                           _P(NttFldsBC), _P(NttGrMatch), C.c_void_p]),
     "ntt_gr_horizon_boundaries": (C.c_int, [_P(NttField), C.c_uint32, C.c_int32, C.c_void_p]),
     "ntt_gr_axis_boundaries": (C.c_int, [_P(NttField), C.c_int32, C.c_uint32, C.c_void_p]),
+    "ntt_gr_field_boundaries": (C.c_int, [_P(NttField), _P(NttField), _P(NttField),
+                                          _P(NttKsMetric), _P(NttFldsBC), _P(NttGrMatch),
+                                          _P(NttGrMatch), C.c_uint32, C.c_int32, C.c_void_p]),
     "ntt_gr_absorb_currents": (C.c_int, [_P(NttField), _P(NttKsMetric), C.c_double, C.c_double,
                                          C.c_int32, C.c_int32, C.c_void_p]),
     "ntt_gr_digital_filter": (C.c_int, [_P(NttField), _P(NttField), _P(NttFldsBC), C.c_void_p]),

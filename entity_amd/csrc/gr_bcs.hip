@@ -70,8 +70,16 @@ struct MatchArgs {
   int      setD, setB, axis_min, axis_max;
 };
 
+// the fields a boundary launch works on, one per blockIdx.y: a GRPIC step
+// applies every boundary to em and em0 alike, so one launch serves both
+struct BPair {
+  BFld f[2];
+  __device__ __forceinline__ const BFld& mine() const { return f[blockIdx.y]; }
+};
+
 template <int KIND>
-__global__ __launch_bounds__(kB) void k_match(BFld F, BFld T, KSMetric<R, KIND> M, MatchArgs a) {
+__global__ __launch_bounds__(kB) void k_match(BPair FF, BFld T, KSMetric<R, KIND> M, MatchArgs a) {
+  const BFld F = FF.mine();
   int i1, i2;
   if (!cell2(a.i1_lo, a.i1_hi, 0, a.N2, i1, i2)) return;
   const R x1 = static_cast<R>(i1 - a.G);
@@ -101,8 +109,9 @@ __global__ __launch_bounds__(kB) void k_match(BFld F, BFld T, KSMetric<R, KIND> 
 
 // Horizon: x1 rows 0 .. 2 + nfilter take row G + 1 + nfilter, x2 rows
 // [G, G + n2]; one thread per x2 row.
-__global__ __launch_bounds__(kB) void k_horizon(BFld F, int G, int n2, int nfilter, int setD,
+__global__ __launch_bounds__(kB) void k_horizon(BPair FF, int G, int n2, int nfilter, int setD,
                                                 int setB) {
+  const BFld F = FF.mine();
   const int i2 = G + static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (i2 > G + n2) return;
   const int src = G + 1 + nfilter;
@@ -115,10 +124,15 @@ __global__ __launch_bounds__(kB) void k_horizon(BFld F, int G, int n2, int nfilt
 
 // Axis rows (one thread per x1 column, ghosts included): the theta
 // components are odd across the axis, the others even; B^theta and D^phi
-// vanish on it.
-__global__ __launch_bounds__(kB) void k_axis(BFld F, int e, int upper, int setD, int setB) {
+// vanish on it.  blockIdx.z: 0 the lower axis, 1 the upper one (their rows are
+// apart for n2 >= 4), from `upper` on.
+__global__ __launch_bounds__(kB) void k_axis(BPair FF, int G, int n2, int upper0, int setD,
+                                             int setB) {
+  const BFld F = FF.mine();
   const int i1 = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (i1 >= F.N1) return;
+  const int upper = upper0 + static_cast<int>(blockIdx.z);
+  const int e = upper ? G + n2 : G;
   if (!upper) {
     if (setD) {
       F.at(i1, e - 1, 1) = -F.at(i1, e, 1);
@@ -358,6 +372,65 @@ ntt_status view2(const ntt_field_t* f, int ncomp, const ntt_ks_metric_t* metric,
 
 using namespace ntt;
 
+namespace {
+
+// one field, or two that the boundaries act on alike (nf = 2)
+BPair pair_of(const FieldView* F, int nf) { return BPair{ { bfld(F[0]), bfld(F[nf - 1]) } }; }
+
+ntt_status match_layer(const FieldView* F, int nf, const FieldView& T,
+                       const ntt_ks_metric_t* metric, const ntt_flds_bc_t* bc,
+                       const ntt_gr_match_t* match, hipStream_t st) {
+  if (!(match->ds > 0.0) || (match->comps & ~0x3Fu) != 0) return NTT_ERR_ARG;
+  if (match->i1_lo < 0 || match->i1_hi > F->N1 || match->i1_lo > match->i1_hi) return NTT_ERR_ARG;
+  if (match->i1_lo == match->i1_hi) return NTT_OK;
+  KSConst<R> k;
+  ntt_status s = make_const<R>(metric, &k);
+  if (s != NTT_OK) return s;
+  MatchArgs a;
+  a.r_edge = match->r_edge;
+  a.four_inv_ds = R(4) / match->ds;
+  a.i1_lo = match->i1_lo;
+  a.i1_hi = match->i1_hi;
+  a.G = F->ngh;
+  a.N2 = F->N2;
+  a.comps = match->comps;
+  a.setD = (match->tags & kTagD) != 0;
+  a.setB = (match->tags & kTagB) != 0;
+  a.axis_min = bc != nullptr && bc->bc[1][0] == NTT_FLDS_BC_AXIS;
+  a.axis_max = bc != nullptr && bc->bc[1][1] == NTT_FLDS_BC_AXIS;
+  const dim3  g(blocks2(a.i1_lo, a.i1_hi, 0, a.N2), nf);
+  const BPair P = pair_of(F, nf);
+  if (metric->kind == NTT_METRIC_KERR_SCHILD)
+    k_match<NTT_METRIC_KERR_SCHILD><<<g, kB, 0, st>>>(P, bfld(T), KSMetric<R, NTT_METRIC_KERR_SCHILD>{ k }, a);
+  else if (metric->kind == NTT_METRIC_QKERR_SCHILD)
+    k_match<NTT_METRIC_QKERR_SCHILD><<<g, kB, 0, st>>>(P, bfld(T), KSMetric<R, NTT_METRIC_QKERR_SCHILD>{ k }, a);
+  else
+    k_match<NTT_METRIC_KERR_SCHILD_0><<<g, kB, 0, st>>>(P, bfld(T), KSMetric<R, NTT_METRIC_KERR_SCHILD_0>{ k }, a);
+  return check_launch();
+}
+
+ntt_status horizon_rows(const FieldView* F, int nf, uint32_t tags, int32_t nfilter,
+                        hipStream_t st) {
+  // the copied row G + 1 + nfilter must lie inside the x1 extent
+  if (nfilter < 0 || F->ngh + 1 + nfilter >= F->N1) return NTT_ERR_ARG;
+  const int setD = (tags & kTagD) != 0, setB = (tags & kTagB) != 0;
+  if (!setD && !setB) return NTT_OK;
+  k_horizon<<<dim3(grid_for(F->n2 + 1, kB), nf), kB, 0, st>>>(pair_of(F, nf), F->ngh, F->n2,
+                                                             nfilter, setD, setB);
+  return check_launch();
+}
+
+// axes `lo` .. `hi` (0: lower, 1: upper)
+ntt_status axis_rows(const FieldView* F, int nf, int lo, int hi, uint32_t tags, hipStream_t st) {
+  const int setD = (tags & kTagD) != 0, setB = (tags & kTagB) != 0;
+  if (!setD && !setB) return NTT_OK;
+  k_axis<<<dim3(grid_for(F->N1, kB), nf, hi - lo + 1), kB, 0, st>>>(pair_of(F, nf), F->ngh, F->n2,
+                                                                    lo, setD, setB);
+  return check_launch();
+}
+
+}  // namespace
+
 extern "C" ntt_status ntt_gr_match_boundaries(ntt_field_t* em, const ntt_field_t* target,
                                               const ntt_ks_metric_t* metric,
                                               const ntt_flds_bc_t* bc, const ntt_gr_match_t* match,
@@ -367,32 +440,7 @@ extern "C" ntt_status ntt_gr_match_boundaries(ntt_field_t* em, const ntt_field_t
   ntt_status s = view2(em, 6, metric, &F);
   if (s != NTT_OK) return s;
   if ((s = view2(target, 6, metric, &T)) != NTT_OK) return s;
-  if (!(match->ds > 0.0) || (match->comps & ~0x3Fu) != 0) return NTT_ERR_ARG;
-  if (match->i1_lo < 0 || match->i1_hi > F.N1 || match->i1_lo > match->i1_hi) return NTT_ERR_ARG;
-  if (match->i1_lo == match->i1_hi) return NTT_OK;
-  KSConst<R> k;
-  if ((s = make_const<R>(metric, &k)) != NTT_OK) return s;
-  MatchArgs a;
-  a.r_edge = match->r_edge;
-  a.four_inv_ds = R(4) / match->ds;
-  a.i1_lo = match->i1_lo;
-  a.i1_hi = match->i1_hi;
-  a.G = F.ngh;
-  a.N2 = F.N2;
-  a.comps = match->comps;
-  a.setD = (match->tags & kTagD) != 0;
-  a.setB = (match->tags & kTagB) != 0;
-  a.axis_min = bc != nullptr && bc->bc[1][0] == NTT_FLDS_BC_AXIS;
-  a.axis_max = bc != nullptr && bc->bc[1][1] == NTT_FLDS_BC_AXIS;
-  const unsigned g = blocks2(a.i1_lo, a.i1_hi, 0, a.N2);
-  hipStream_t st = as_stream(stream);
-  if (metric->kind == NTT_METRIC_KERR_SCHILD)
-    k_match<NTT_METRIC_KERR_SCHILD><<<g, kB, 0, st>>>(bfld(F), bfld(T), KSMetric<R, NTT_METRIC_KERR_SCHILD>{ k }, a);
-  else if (metric->kind == NTT_METRIC_QKERR_SCHILD)
-    k_match<NTT_METRIC_QKERR_SCHILD><<<g, kB, 0, st>>>(bfld(F), bfld(T), KSMetric<R, NTT_METRIC_QKERR_SCHILD>{ k }, a);
-  else
-    k_match<NTT_METRIC_KERR_SCHILD_0><<<g, kB, 0, st>>>(bfld(F), bfld(T), KSMetric<R, NTT_METRIC_KERR_SCHILD_0>{ k }, a);
-  return check_launch();
+  return match_layer(&F, 1, T, metric, bc, match, as_stream(stream));
 }
 
 extern "C" ntt_status ntt_gr_horizon_boundaries(ntt_field_t* em, uint32_t tags, int32_t nfilter,
@@ -400,13 +448,7 @@ extern "C" ntt_status ntt_gr_horizon_boundaries(ntt_field_t* em, uint32_t tags, 
   FieldView F;
   ntt_status s = view2(em, 6, nullptr, &F);
   if (s != NTT_OK) return s;
-  // the copied row G + 1 + nfilter must lie inside the x1 extent
-  if (nfilter < 0 || F.ngh + 1 + nfilter >= F.N1) return NTT_ERR_ARG;
-  const int setD = (tags & kTagD) != 0, setB = (tags & kTagB) != 0;
-  if (!setD && !setB) return NTT_OK;
-  k_horizon<<<grid_for(F.n2 + 1, kB), kB, 0, as_stream(stream)>>>(bfld(F), F.ngh, F.n2, nfilter,
-                                                                   setD, setB);
-  return check_launch();
+  return horizon_rows(&F, 1, tags, nfilter, as_stream(stream));
 }
 
 extern "C" ntt_status ntt_gr_axis_boundaries(ntt_field_t* em, int32_t upper, uint32_t tags,
@@ -414,11 +456,50 @@ extern "C" ntt_status ntt_gr_axis_boundaries(ntt_field_t* em, int32_t upper, uin
   FieldView F;
   ntt_status s = view2(em, 6, nullptr, &F);
   if (s != NTT_OK) return s;
-  const int setD = (tags & kTagD) != 0, setB = (tags & kTagB) != 0;
-  if (!setD && !setB) return NTT_OK;
-  const int e = upper ? F.ngh + F.n2 : F.ngh;
-  k_axis<<<grid_for(F.N1, kB), kB, 0, as_stream(stream)>>>(bfld(F), e, upper ? 1 : 0, setD, setB);
-  return check_launch();
+  return axis_rows(&F, 1, upper ? 1 : 0, upper ? 1 : 0, tags, as_stream(stream));
+}
+
+extern "C" ntt_status ntt_gr_field_boundaries(ntt_field_t* em, ntt_field_t* em0,
+                                              const ntt_field_t* target,
+                                              const ntt_ks_metric_t* metric,
+                                              const ntt_flds_bc_t* bc,
+                                              const ntt_gr_match_t* match_lo,
+                                              const ntt_gr_match_t* match_hi, uint32_t tags,
+                                              int32_t nfilter, void* stream) {
+  if (!metric_kind_ok(metric)) return metric ? NTT_ERR_UNSUPPORTED : NTT_ERR_ARG;
+  if (bc == nullptr) return NTT_ERR_ARG;
+  FieldView  F[2], T{};
+  ntt_status s = view2(em, 6, metric, &F[0]);
+  if (s != NTT_OK) return s;
+  if ((s = view2(em0, 6, metric, &F[1])) != NTT_OK) return s;
+  if (F[0].d == F[1].d) return NTT_ERR_ARG;
+  const uint8_t* x1 = bc->bc[0];
+  const ntt_gr_match_t* m[2] = { match_lo, match_hi };
+  for (int e = 0; e < 2; ++e) {
+    if (bc->bc[1][e] != NTT_FLDS_BC_AXIS) return NTT_ERR_UNSUPPORTED;
+    if (x1[e] == NTT_FLDS_BC_MATCH) {
+      if (m[e] == nullptr) return NTT_ERR_ARG;
+      if ((s = view2(target, 6, metric, &T)) != NTT_OK) return s;
+    } else if (x1[e] != NTT_FLDS_BC_HORIZON) {
+      return NTT_ERR_UNSUPPORTED;
+    }
+  }
+  hipStream_t st = as_stream(stream);
+  // the order of Directions<2D>::orth: -x1, -x2, +x2, +x1
+  auto side = [&](int e) {
+    if (x1[e] == NTT_FLDS_BC_HORIZON) return horizon_rows(F, 2, tags, nfilter, st);
+    ntt_gr_match_t a = *m[e];
+    a.tags = tags;
+    return match_layer(F, 2, T, metric, bc, &a, st);
+  };
+  if ((s = side(0)) != NTT_OK) return s;
+  if (F[0].n2 >= 4) {
+    if ((s = axis_rows(F, 2, 0, 1, tags, st)) != NTT_OK) return s;
+  } else {
+    if ((s = axis_rows(F, 2, 0, 0, tags, st)) != NTT_OK) return s;
+    if ((s = axis_rows(F, 2, 1, 1, tags, st)) != NTT_OK) return s;
+  }
+  return side(1);
 }
 
 extern "C" ntt_status ntt_gr_absorb_currents(ntt_field_t* cur, const ntt_ks_metric_t* metric,

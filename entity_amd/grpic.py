@@ -316,18 +316,15 @@ class GRPICEngine(GRRun):
                 gr.AbsorbCurrents_kernel(self.cur0, self.shape, self.metric, edge,
                                          self.ds[0][1], (lo, hi))(stream)
             return
-        for d, side in ((0, 0), (1, 0), (1, 1), (0, 1)):   # Directions<2D>::orth
-            bc = self.flds_bc[d][side]
-            for F in (self.em, self.em0):
-                if bc == _abi.FLDS_BC_MATCH:
-                    lo, hi, edge = self._layers[side]
-                    gr.MatchBoundaries_kernel(F, self.target, self.shape, self.metric, edge,
-                                              self.ds[0][side], tags, (lo, hi), self.comps,
-                                              self._bcs())(stream)
-                elif bc == _abi.FLDS_BC_AXIS:
-                    gr.AxisBoundaries_kernel(F, self.shape, side == 1, tags)(stream)
-                elif bc == _abi.FLDS_BC_HORIZON:
-                    gr.HorizonBoundaries_kernel(F, self.shape, tags, self.nfilter)(stream)
+        # em and em0 together, in the order of Directions<2D>::orth
+        m = [_abi.NttGrMatch(edge, self.ds[0][side], lo, hi, tags, self.comps)
+             for side in (0, 1) for lo, hi, edge in (self._layers[side],)]
+        f, f0, t = (field_abi(x, self.shape) for x in (self.em, self.em0, self.target))
+        bc = gr._Field._bc(self._bcs())
+        _abi.check(self.lib.ntt_gr_field_boundaries(
+            C.byref(f), C.byref(f0), C.byref(t), C.byref(self.metric.abi()), C.byref(bc),
+            C.byref(m[0]), C.byref(m[1]), tags, self.nfilter, _stream(stream)),
+            "ntt_gr_field_boundaries")
 
     def _aux_e(self, D, B, st):
         gr.ComputeAuxE_kernel(D, B, self.aux, self.shape, self.metric, self._bcs())(st)

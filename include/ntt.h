@@ -360,6 +360,20 @@ NTT_API ntt_status ntt_gr_horizon_boundaries(ntt_field_t* em, uint32_t tags, int
 NTT_API ntt_status ntt_gr_axis_boundaries(ntt_field_t* em, int32_t upper, uint32_t tags,
                                           void* stream);
 
+/* The field boundaries of a GRPIC step on em and em0 together, in the order of
+ * the reference's directions (-x1, -x2, +x2, +x1): per x1 side of bc MATCH
+ * (match_lo / match_hi as in ntt_gr_match_boundaries, with `tags` in place of
+ * theirs) or HORIZON, and AXIS on both x2 sides.  Equal to the three calls
+ * above on each field, in three launches instead of eight.  Replaces
+ * grpic::FieldBoundaries (src/engines/grpic/fields_bcs.h:234-266) for one
+ * domain. */
+NTT_API ntt_status ntt_gr_field_boundaries(ntt_field_t* em, ntt_field_t* em0,
+                                           const ntt_field_t* target,
+                                           const ntt_ks_metric_t* metric, const ntt_flds_bc_t* bc,
+                                           const ntt_gr_match_t* match_lo,
+                                           const ntt_gr_match_t* match_hi, uint32_t tags,
+                                           int32_t nfilter, void* stream);
+
 /* J *= tanh(|r(x1) - r_edge| / (ds / 4)) over x1 cells [i1_lo, i1_hi), every
  * x2 row.  Replaces kernel::bc::gr::AbsorbCurrents_kernel
  * (src/kernels/fields_bcs.hpp:1243-1280). */

@@ -287,6 +287,203 @@ struct KSMetric {
   }
 };
 
+// ---- FP64 points of the Kerr-Schild and quasi-spherical metrics ---------------
+// The metric's formulas regrouped around one reciprocal per point, with
+// reciprocals and reciprocal roots from the hardware estimate and two Newton
+// steps (about 1 ulp) in the place of IEEE divisions and roots.  A point a
+// fraction of a cell away from another takes its exp, sin and cos from that
+// one's by the addition theorems.
+__device__ __forceinline__ double rcp64(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
+}
+__device__ __forceinline__ double rsq64(double x) {
+  double y = __builtin_amdgcn_rsq(x), g = x * y, h = 0.5 * y;
+  double d = fma(-h, g, 0.5);
+  g = fma(g, d, g);
+  h = fma(h, d, h);
+  d = fma(-h, g, 0.5);
+  h = fma(h, d, h);
+  return 2.0 * h;
+}
+
+// exp(d) - sin(d), cos(d) for |d| up to kNear: Taylor, truncated below 2e-17
+constexpr double kNear = 0.03;
+__device__ __forceinline__ double exp_near(double d) {
+  double p = fma(d, 1.0 / 5040, 1.0 / 720);
+  p = fma(d, p, 1.0 / 120);
+  p = fma(d, p, 1.0 / 24);
+  p = fma(d, p, 1.0 / 6);
+  p = fma(d, p, 0.5);
+  p = fma(d, p, 1.0);
+  return fma(d, p, 1.0);
+}
+__device__ __forceinline__ void sin_cos_near(double d, double* s, double* c) {
+  const double q = d * d;
+  double p = fma(q, -1.0 / 5040, 1.0 / 120);
+  p  = fma(q, p, -1.0 / 6);
+  *s = fma(d * q, p, d);
+  p  = fma(q, 1.0 / 40320, -1.0 / 720);
+  p  = fma(q, p, 1.0 / 24);
+  p  = fma(q, p, -0.5);
+  *c = fma(q, p, 1.0);
+}
+
+template <int KIND>
+struct FastPoint {
+  double th, s, c, e;        // theta, its sine and cosine, exp(chi) (quasi-spherical)
+  double r, s2, S, P, Dl, A; // P = Sigma + 2 r
+  double iS, iP, iSP, iSs2;  // 1 / S, 1 / P, 1 / (S P), 1 / (S sin^2)
+  double g, gi;              // 1 / (dr/dx1), dr/dx1
+  double ti, ith;            // dtheta/dx2 and its reciprocal
+  double h11, h22, h33, h13, beta1;
+
+  // everything that follows from r, s, c, e and dtheta/dx2
+  __device__ __forceinline__ void finish(const KSMetric<double, KIND>& M) {
+    const double a2 = sqr(M.k.a);
+    s2 = sqr(s);
+    S  = sqr(r) + a2 * sqr(c);
+    P  = S + 2.0 * r;
+    Dl = sqr(r) - 2.0 * r + a2;
+    A  = sqr(sqr(r) + a2) - a2 * Dl * s2;
+    const double SP = S * P, q = SP * s2;
+    double       t;  // 1 / (S P sin^2)
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      const double T = rcp64(q * e);
+      t  = T * e;
+      g  = T * q * M.k.dchi_inv;
+      gi = M.k.dchi * e;
+    } else {
+      t  = rcp64(q);
+      g  = M.k.dr_inv;
+      gi = M.k.dr;
+    }
+    iSs2  = t * P;
+    iS    = iSs2 * s2;
+    iSP   = t * s2;
+    iP    = iSP * S;
+    h11   = sqr(g) * A * iSP;
+    h22   = sqr(ith) * iS;
+    h33   = iSs2;
+    h13   = g * M.k.a * iS;
+    beta1 = g * (2.0 * r) * iP;
+  }
+  __device__ __forceinline__ void angle_scale(const KSMetric<double, KIND>& M, double eta) {
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      ti  = M.k.deta;
+      ith = M.k.deta_inv;
+      if (!almost_zero(M.k.h0)) {
+        const double f = M.dtheta_deta(eta);
+        ti *= f;
+        ith *= rcp64(f);
+      }
+    } else {
+      ti  = M.k.dtheta;
+      ith = M.k.dtheta_inv;
+    }
+  }
+  // at code coordinates (x1, x2)
+  __device__ __forceinline__ void at(const KSMetric<double, KIND>& M, double x1, double x2) {
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      e = exp(x1 * M.k.dchi + M.k.chi_min);
+      r = M.k.r0 + e;
+      angle_scale(M, x2 * M.k.deta + M.k.eta_min);
+    } else {
+      e = 0.0;
+      r = x1 * M.k.dr + M.k.x1_min;
+      angle_scale(M, 0.0);
+    }
+    th = M.theta_ph(x2);
+    sin_cos(th, &s, &c);
+    finish(M);
+  }
+  // at (x1, x2), starting from the point b at (b1, .)
+  __device__ __forceinline__ void near(const KSMetric<double, KIND>& M, const FastPoint& b,
+                                       double b1, double x1, double x2) {
+    th = M.theta_ph(x2);
+    const double dth = th - b.th;
+    double       dchi = 0.0;
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) dchi = (x1 - b1) * M.k.dchi;
+    if (fabs(dth) <= kNear && fabs(dchi) <= kNear) {
+      double sd, cd;
+      sin_cos_near(dth, &sd, &cd);
+      s = fma(b.c, sd, b.s * cd);
+      c = fma(-b.s, sd, b.c * cd);
+      if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) e = b.e * exp_near(dchi);
+    } else {
+      sin_cos(th, &s, &c);
+      if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) e = exp(x1 * M.k.dchi + M.k.chi_min);
+    }
+    if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) {
+      r = M.k.r0 + e;
+      angle_scale(M, x2 * M.k.deta + M.k.eta_min);
+    } else {
+      e = 0.0;
+      r = x1 * M.k.dr + M.k.x1_min;
+      angle_scale(M, 0.0);
+    }
+    finish(M);
+  }
+  __device__ __forceinline__ double alpha() const { return rsq64(P * iS); }
+  __device__ __forceinline__ void to_cntrv(const double* v, double* u) const {
+    u[0] = v[0] * h11 + v[2] * h13;
+    u[1] = v[1] * h22;
+    u[2] = v[0] * h13 + v[2] * h33;
+  }
+  // KSMetric::derivs at this point, the same quirks
+  __device__ __forceinline__ void derivs(const KSMetric<double, KIND>& M, double x2, double al,
+                                         typename KSMetric<double, KIND>::Deriv& d) const {
+    constexpr bool Q  = KIND == NTT_METRIC_QKERR_SCHILD;
+    const double   a  = M.k.a, a2 = sqr(a);
+    const double   iS2 = sqr(iS), al3 = cube(al), g2 = sqr(g);
+    const double   dr_S = 2.0 * r * gi;
+    double dth2;  // the angle's derivative that dt_S and dt_A use
+    double dt_S0; // dt_S without the cut of tiny values, for dt_alpha
+    double i22;   // the angle factor of the derivatives of h^22
+    if constexpr (Q) {
+      const double eta = x2 * M.k.deta + M.k.eta_min;
+      dth2 = M.dx_dt(eta);
+      // dt_alpha uses the stretching derivative without the AlmostZero cuts
+      dt_S0 = -2.0 * a2 * s * c *
+              (M.k.deta * (1.0 + 2.0 * M.k.h0 * kInvPiSqr *
+                                   (6.0 * sqr(eta) - 6.0 * kPi * eta + kPiSqr)));
+      i22 = sqr(M.k.deta_inv);
+    } else {
+      dth2  = M.k.dtheta;
+      dt_S0 = 0.0;
+      i22   = sqr(M.k.dtheta_inv);
+    }
+    double dt_S = -2.0 * a2 * s * c * dth2, dt_A = dt_S * Dl;
+    if (almost_zero(dt_S)) dt_S = 0.0;
+    if (almost_zero(dt_A)) dt_A = 0.0;
+    if constexpr (!Q) dt_S0 = dt_S;
+    const double dr_D = 2.0 * gi * (r - 1.0);
+    const double dr_A = 4.0 * r * gi * (sqr(r) + a2) - a2 * s2 * dr_D;
+    const double dSr  = gi * S - r * dr_S;
+    const double iSP2 = sqr(iSP), SS = S * P, iP2 = sqr(iP);
+    d.dr_alpha = -dSr * al3 * iS2;
+    d.dt_alpha = r * dt_S0 * al3 * iS2;
+    d.dr_beta1 = 2.0 * g * dSr * iP2;
+    d.dt_beta1 = -2.0 * g * r * dt_S * iP2;
+    d.dr_h11   = g2 * (SS * dr_A - 2.0 * A * (r * dr_S + S * (dr_S + gi))) * iSP2;
+    d.dr_h22   = -dr_S * iS2 * i22;
+    d.dr_h33   = -dr_S * iS * iSs2;
+    d.dr_h13   = -a * dr_S * iS2 * g;
+    d.dt_h11   = g2 * (SS * dt_A - 2.0 * A * dt_S * (r + S)) * iSP2;
+    d.dt_h22   = -dt_S * iS2 * i22;
+    d.dt_h13   = -a * dt_S * iS2 * g;
+    if constexpr (Q) {
+      d.dr_beta1 -= M.k.dchi * beta1;
+      d.dr_h11 -= 2.0 * M.k.dchi * h11;
+      d.dr_h13 -= M.k.dchi * h13;
+      d.dt_h33 = -(dt_S * s + 2.0 * c * S * dth2) * sqr(iSs2) * s;
+    } else {
+      d.dt_h33 = -2.0 * M.k.dtheta * c * (S - a2 * s2) * sqr(iSs2) * s;
+    }
+  }
+};
+
 // host: metric constants in R, as the reference's metric constructors
 // compute them (kerr_schild.h:79-90, qkerr_schild.h:79-94)
 template <typename R>

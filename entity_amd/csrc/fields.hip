@@ -180,44 +180,52 @@ __global__ __launch_bounds__(BX* BY) void k_filter_2d(FieldView A, FieldView B) 
   }
 }
 
-// 3D: the 1/32 group is the reference's list as written (it names
-// (i,j,k-1) and (i,j,k+1) where the edge pair (i,j-1,k+1), (i,j+1,k-1) would
-// complete the binomial stencil).
-__global__ __launch_bounds__(BX* BY) void k_filter_3d(FieldView A, FieldView B) {
-  const CellIdx c = active_cell(A);
-  if (!c.ok) return;
-  const int i = c.i, j = c.j, k = c.k;
-#pragma unroll
-  for (int comp = 0; comp < 3; ++comp) {
-    auto b = [&](int x, int y, int z) -> float { return B(x, y, z, comp); };
-    A(i, j, k, comp) =
-      INV_8 * b(i, j, k) +
-      INV_16 * (b(i - 1, j, k) + b(i + 1, j, k) + b(i, j - 1, k) + b(i, j + 1, k) + b(i, j, k - 1) +
-                b(i, j, k + 1)) +
-      INV_32 * (b(i - 1, j - 1, k) + b(i + 1, j + 1, k) + b(i - 1, j + 1, k) + b(i + 1, j - 1, k) +
-                b(i, j - 1, k - 1) + b(i, j + 1, k + 1) + b(i, j, k - 1) + b(i, j, k + 1) +
-                b(i - 1, j, k - 1) + b(i + 1, j, k + 1) + b(i - 1, j, k + 1) + b(i + 1, j, k - 1)) +
-      INV_64 * (b(i - 1, j - 1, k - 1) + b(i + 1, j + 1, k + 1) + b(i - 1, j + 1, k + 1) +
-                b(i + 1, j - 1, k - 1) + b(i - 1, j - 1, k + 1) + b(i + 1, j + 1, k - 1) +
-                b(i - 1, j + 1, k - 1) + b(i + 1, j - 1, k + 1));
-  }
-}
-
 // ---- periodic ghost fill: metadomain_comm.cpp:204-367 -----------------------
 __device__ __forceinline__ int wrap_src(int i, int G, int n) {
   return i < G ? i + n : (i >= G + n ? i - n : i);
 }
 
-__global__ __launch_bounds__(BX* BY) void k_ghost_fill(FieldView F, int c0, int c1) {
-  const int i = blockIdx.x * BX + threadIdx.x;
-  const int j = blockIdx.y * BY + threadIdx.y;
-  const int k = blockIdx.z;
-  if (i >= F.N1 || j >= F.N2) return;
-  const int G  = F.ngh;
+// One thread per ghost cell: the 2 G planes below and above along z, the 2 G
+// rows of the active planes along y, the 2 G cells of their active rows along
+// x.  (A thread for every cell of the array, most of which had nothing to do,
+// took 19 us at 250 x 156 x 131 cells and three components; the shell 6.5 us.)
+struct Shell {
+  int64_t nz, ny, nx;  // ghost cells of the three parts
+};
+__host__ __device__ __forceinline__ Shell shell_of(const FieldView& F) {
+  const int64_t g2 = 2 * F.ngh, n3 = F.N3 > 1 ? F.n3 : 1;
+  return Shell{ F.N3 > 1 ? g2 * F.N1 * F.N2 : 0, n3 * g2 * F.N1, n3 * F.n2 * g2 };
+}
+
+constexpr int kGhostBlock = 256;
+__global__ __launch_bounds__(kGhostBlock) void k_ghost_fill(FieldView F, int c0, int c1) {
+  const Shell S = shell_of(F);
+  int64_t     t = static_cast<int64_t>(blockIdx.x) * kGhostBlock + threadIdx.x;
+  const int   G = F.ngh, G2 = 2 * G;
+  // index along a dimension of the q-th ghost layer
+  auto layer = [&](int q, int n) { return q < G ? q : n + q; };
+  int i, j, k = 0;
+  if (t < S.nz) {
+    i = static_cast<int>(t % F.N1);
+    t /= F.N1;
+    j = static_cast<int>(t % F.N2);
+    k = layer(static_cast<int>(t / F.N2), F.n3);
+  } else if ((t -= S.nz) < S.ny) {
+    i = static_cast<int>(t % F.N1);
+    t /= F.N1;
+    j = layer(static_cast<int>(t % G2), F.n2);
+    if (F.N3 > 1) k = static_cast<int>(t / G2) + G;
+  } else if ((t -= S.ny) < S.nx) {
+    i = layer(static_cast<int>(t % G2), F.n1);
+    t /= G2;
+    j = static_cast<int>(t % F.n2) + G;
+    if (F.N3 > 1) k = static_cast<int>(t / F.n2) + G;
+  } else {
+    return;
+  }
   const int si = wrap_src(i, G, F.n1);
   const int sj = wrap_src(j, G, F.n2);
   const int sk = (F.N3 > 1) ? wrap_src(k, G, F.n3) : k;
-  if (si == i && sj == j && sk == k) return;
   for (int comp = c0; comp < c1; ++comp) F(i, j, k, comp) = F(si, sj, sk, comp);
 }
 
@@ -425,6 +433,11 @@ constexpr int FHX = FTX + 2, FHY = FTY + 2, FPL = FHX * FHY;
 // overlaps it, and are written to the ring after.
 constexpr int FLD = (3 * FPL + FTX * FTY - 1) / (FTX * FTY);
 
+// GHOSTS: the destination's ghost copies are written too (the engine's pass);
+// without, only the active cells (ntt_digital_filter, whose one thread per cell
+// reading 81 values through the caches took 66 us at 250 x 156 x 131 cells:
+// 45 us here).
+template <bool GHOSTS>
 __global__ __launch_bounds__(FTX* FTY) void k_filter_periodic_3d(FieldView Dst, FieldView Src) {
   __shared__ float ring[3][3 * FPL];
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * FTX + tx;
@@ -485,11 +498,18 @@ __global__ __launch_bounds__(FTX* FTY) void k_filter_periodic_3d(FieldView Dst, 
           for (int y = 0; y < 3; ++y)
 #pragma unroll
             for (int x = 0; x < 3; ++x) b[z][y][x] = pl[z][o + (y - 1) * FHX + (x - 1)];
-        store_with_ghosts(Dst, i + G, j + G, k + G, comp, filter3d_value(b));
+        if constexpr (GHOSTS) store_with_ghosts(Dst, i + G, j + G, k + G, comp, filter3d_value(b));
+        else Dst(i + G, j + G, k + G, comp) = filter3d_value(b);
       }
     }
     __syncthreads();
   }
+}
+
+template <bool GHOSTS>
+void launch_filter_3d(const FieldView& dst, const FieldView& src, hipStream_t st) {
+  const dim3 grid((dst.n1 + FTX - 1) / FTX, (dst.n2 + FTY - 1) / FTY, (dst.n3 + FKC - 1) / FKC);
+  k_filter_periodic_3d<GHOSTS><<<grid, dim3(FTX, FTY), 0, st>>>(dst, src);
 }
 
 __global__ void k_fill_zero(float* __restrict__ d, int64_t n) {
@@ -660,7 +680,7 @@ extern "C" ntt_status ntt_digital_filter(ntt_field_t* array, const ntt_field_t* 
         if (bc->bc[d][e] != NTT_FLDS_BC_PERIODIC) return NTT_ERR_UNSUPPORTED;
   }
   if (array->dim == 2) k_filter_2d<<<active_grid(A), dim3(BX, BY), 0, as_stream(stream)>>>(A, B);
-  else k_filter_3d<<<active_grid(A), dim3(BX, BY), 0, as_stream(stream)>>>(A, B);
+  else launch_filter_3d<false>(A, B, as_stream(stream));
   return launch_ok();
 }
 
@@ -671,8 +691,7 @@ extern "C" ntt_status ntt_communicate_fields(ntt_field_t* fld, int32_t comp_begi
   if (s != NTT_OK) return s;
   if (comp_begin < 0 || comp_end > F.nc || comp_begin >= comp_end) return NTT_ERR_ARG;
   if (F.n1 < F.ngh || F.n2 < F.ngh || (F.N3 > 1 && F.n3 < F.ngh)) return NTT_ERR_ARG;
-  const dim3 grid((F.N1 + BX - 1) / BX, (F.N2 + BY - 1) / BY, F.N3);
-  k_ghost_fill<<<grid, dim3(BX, BY), 0, as_stream(stream)>>>(F, comp_begin, comp_end);
+  launch_ghost_fill(F, comp_begin, comp_end, as_stream(stream));
   return launch_ok();
 }
 
@@ -708,16 +727,15 @@ void launch_ampere_currents_periodic(const FieldView& F, const FieldView& J, flo
 
 void launch_filter_periodic(const FieldView& dst, const FieldView& src, hipStream_t st) {
   if (dst.N3 > 1) {
-    const dim3 grid((dst.n1 + FTX - 1) / FTX, (dst.n2 + FTY - 1) / FTY, (dst.n3 + FKC - 1) / FKC);
-    k_filter_periodic_3d<<<grid, dim3(FTX, FTY), 0, st>>>(dst, src);
+    launch_filter_3d<true>(dst, src, st);
     return;
   }
   k_filter_periodic<<<active_grid(dst), dim3(BX, BY), 0, st>>>(dst, src);
 }
 
 void launch_ghost_fill(const FieldView& F, int c0, int c1, hipStream_t st) {
-  const dim3 grid((F.N1 + BX - 1) / BX, (F.N2 + BY - 1) / BY, F.N3);
-  k_ghost_fill<<<grid, dim3(BX, BY), 0, st>>>(F, c0, c1);
+  const Shell S = shell_of(F);
+  k_ghost_fill<<<grid_for(S.nz + S.ny + S.nx, kGhostBlock), kGhostBlock, 0, st>>>(F, c0, c1);
 }
 
 void launch_fold(const FieldView& J, hipStream_t st) {

@@ -245,9 +245,14 @@ ntt_status sr_step(ntt_field_t* em, ntt_field_t* cur, ntt_field_t* buff, ntt_spe
   // srpic.hpp:71-82: fill E and B ghosts at step 0
   if (prm->step == 0) launch_ghost_fill(E, 0, 6, st);
 
-  auto faraday_half = [&]() -> ntt_status {
+  // currents.h:68: J = 0 -- here the fixed-point accumulator, cleared by the
+  // launch of the first Faraday half where there is one (a kernel rather than
+  // a memset, so that the step can be captured in a graph)
+  const bool clear_first = prm->deposit_enable && prm->fieldsolver_enable && !P.ext;
+  auto faraday_half = [&](bool first) -> ntt_status {
     if (!P.ext) {
-      launch_faraday_periodic(E, P.far_c1, P.far_c2, st);
+      launch_faraday_periodic(E, P.far_c1, P.far_c2, st,
+                              first && clear_first ? P.acc : nullptr, J.cstride * 3);
       return check_launch();
     }
     ntt_status r = ntt_faraday_mink(em, P.far_c1, P.far_c2, &prm->fd, stream);
@@ -257,14 +262,12 @@ ntt_status sr_step(ntt_field_t* em, ntt_field_t* cur, ntt_field_t* buff, ntt_spe
   };
 
   if (prm->fieldsolver_enable) {
-    s = faraday_half();
+    s = faraday_half(true);
     if (s != NTT_OK) return s;
   }
   // the fields the push gathers, for a caller that records them
   if (prm->em_half_out != nullptr) launch_copy(prm->em_half_out, E.d, E.cstride * 6, st);
-  // currents.h:68: J = 0 -- here the fixed-point accumulator (a fill kernel
-  // rather than a memset, so that the step can be captured in a graph)
-  if (prm->deposit_enable) launch_zero_u64(P.acc, J.cstride * 3, st);
+  if (prm->deposit_enable && !clear_first) launch_zero_u64(P.acc, J.cstride * 3, st);
   {
     std::vector<SpeciesPush> push;
     push.reserve(nspecies);
@@ -287,23 +290,12 @@ ntt_status sr_step(ntt_field_t* em, ntt_field_t* cur, ntt_field_t* buff, ntt_spe
     if (s != NTT_OK) return s;
   }
   if (prm->deposit_enable) {
-    // folded current (active cells + periodic ghosts) from the accumulator
-    launch_j_from_fixed(J, P.acc, 1.0 / static_cast<double>(P.fscale), st);
-    // currents.h:89-119: n filter passes (ping-pong between cur and buff)
-    if (prm->n_filters > 0) {
-      const FieldView* src = &J;
-      const FieldView* dst = &Bf;
-      for (int f = 0; f < prm->n_filters; ++f) {
-        launch_filter_periodic(*dst, *src, st);
-        const FieldView* t = src;
-        src = dst;
-        dst = t;
-      }
-      if (src != &J) launch_copy(J.d, Bf.d, J.cstride * 3, st);
-    }
+    // folded current (active cells + periodic ghosts) from the accumulator, and
+    // its filter passes (currents.h:89-119)
+    launch_filtered_current(J, Bf, P.acc, 1.0 / static_cast<double>(P.fscale), prm->n_filters, st);
   }
   if (prm->fieldsolver_enable) {
-    s = faraday_half();
+    s = faraday_half(false);
     if (s != NTT_OK) return s;
     launch_ampere_currents_periodic(E, J, P.amp_c1, P.amp_c2, P.amp_coeff, prm->ppc0,
                                     prm->deposit_enable != 0, st);
@@ -381,7 +373,7 @@ struct ntt_ensemble {
     int64_t blocks;
   };
   std::vector<FieldView> ghost_E;   // step 0: E/B ghost fill per box
-  Seg                    far, zero, jfix, amp, copy;
+  Seg                    far, zero, jfix, amp;
   // batched tile re-sort of every (box, species) whose box names a tile
   Seg                    sort;      // device SortSeg[n]
   int64_t*               sort_pbase = nullptr;
@@ -428,9 +420,9 @@ extern "C" ntt_status ntt_ensemble_create(const ntt_box_t* boxes, int32_t nboxes
   ntt_ensemble* e = new ntt_ensemble();
   (void)hipGetDevice(&e->device);
   std::vector<FieldSeg> far, jfix, amp;
-  std::vector<FlatSeg>  zero, copy;
+  std::vector<FlatSeg>  zero;
   std::vector<std::vector<FieldSeg>> passes;
-  int64_t nb_far = 0, nb_jfix = 0, nb_amp = 0, nb_zero = 0, nb_copy = 0;
+  int64_t nb_far = 0, nb_jfix = 0, nb_amp = 0, nb_zero = 0;
   std::vector<int64_t> nb_pass;
   struct GroupHost {
     int D, order, alg;
@@ -477,19 +469,20 @@ extern "C" ntt_status ntt_ensemble_create(const ntt_box_t* boxes, int32_t nboxes
     }
     if (prm.deposit_enable) {
       const int64_t n = P.J.cstride * 3;
-      zero.push_back(FlatSeg{ P.acc, nullptr, n, nb_zero });
+      zero.push_back(FlatSeg{ P.acc, n, nb_zero });
       nb_zero += flat_seg_blocks(n);
+      // the current and its filter passes alternate between J and Bf so that
+      // the last one writes J
+      const FieldView* dst[2] = { &P.J, &P.Bf };
       FieldSeg j{};
       j.gx = gx;
       j.gy = gy;
-      j.F = P.J;
+      j.F = *dst[prm.n_filters % 2];
       j.acc = P.acc;
       j.inv_scale = 1.0 / static_cast<double>(P.fscale);
       j.blk0 = nb_jfix;
       jfix.push_back(j);
       nb_jfix += nblk;
-      const FieldView* src = &P.J;
-      const FieldView* dst = &P.Bf;
       for (int f = 0; f < prm.n_filters; ++f) {
         if (static_cast<int>(passes.size()) <= f) {
           passes.emplace_back();
@@ -498,16 +491,11 @@ extern "C" ntt_status ntt_ensemble_create(const ntt_box_t* boxes, int32_t nboxes
         FieldSeg q{};
         q.gx = gx;
         q.gy = gy;
-        q.F = *dst;
-        q.J = *src;
+        q.F = *dst[(prm.n_filters - f - 1) % 2];
+        q.J = *dst[(prm.n_filters - f) % 2];
         q.blk0 = nb_pass[f];
         passes[f].push_back(q);
         nb_pass[f] += nblk;
-        std::swap(src, dst);
-      }
-      if (src != &P.J) {
-        copy.push_back(FlatSeg{ P.J.d, P.Bf.d, n, nb_copy });
-        nb_copy += flat_seg_blocks(n);
       }
     }
     if (B.tile[0] > 0) {
@@ -563,7 +551,6 @@ extern "C" ntt_status ntt_ensemble_create(const ntt_box_t* boxes, int32_t nboxes
   if (s == NTT_OK) s = upload_segs(e, amp, nb_amp, &e->amp);
   if (s == NTT_OK) s = upload_segs(e, jfix, nb_jfix, &e->jfix);
   if (s == NTT_OK) s = upload_segs(e, zero, nb_zero, &e->zero);
-  if (s == NTT_OK) s = upload_segs(e, copy, nb_copy, &e->copy);
   for (size_t f = 0; f < passes.size() && s == NTT_OK; ++f) {
     ntt_ensemble::Seg seg;
     s = upload_segs(e, passes[f], nb_pass[f], &seg);
@@ -621,11 +608,8 @@ extern "C" ntt_status ntt_ensemble_step(ntt_ensemble_t e, int64_t step, void* st
   auto fields = [&](int op, const ntt_ensemble::Seg& sg) {
     launch_fields_batched(op, static_cast<const FieldSeg*>(sg.dev), sg.n, sg.blocks, st);
   };
-  auto flat = [&](int op, const ntt_ensemble::Seg& sg) {
-    launch_flat_batched(op, static_cast<const FlatSeg*>(sg.dev), sg.n, sg.blocks, st);
-  };
   fields(SEG_FARADAY, e->far);
-  flat(FLAT_ZERO_U64, e->zero);
+  launch_zero_batched(static_cast<const FlatSeg*>(e->zero.dev), e->zero.n, e->zero.blocks, st);
   for (const auto& g : e->groups) {
     ntt_status s = launch_push_deposit_batched(g.D, g.order, g.alg, g.table, g.chunk0, g.nent,
                                                g.nchunks, st);
@@ -633,7 +617,6 @@ extern "C" ntt_status ntt_ensemble_step(ntt_ensemble_t e, int64_t step, void* st
   }
   fields(SEG_JFIX, e->jfix);
   for (const auto& p : e->filter_pass) fields(SEG_FILTER, p);
-  flat(FLAT_COPY_F32, e->copy);
   fields(SEG_FARADAY, e->far);
   fields(SEG_AMPERE, e->amp);
   return check_launch();

@@ -57,7 +57,9 @@ float fixed_point_scale(float qw_max, float dt);
 float fixed_point_small_coeff(float dt);
 
 // fields.hip
-void launch_faraday_periodic(const FieldView& F, float c1, float c2, hipStream_t st);
+// clear: nclear 64-bit entries to clear in the same launch (null: none)
+void launch_faraday_periodic(const FieldView& F, float c1, float c2, hipStream_t st,
+                             unsigned long long* clear = nullptr, int64_t nclear = 0);
 void launch_ampere_currents_periodic(const FieldView& F, const FieldView& J, float c1, float c2,
                                      float coeff, float ppc0, bool with_j, hipStream_t st);
 void launch_filter_periodic(const FieldView& dst, const FieldView& src, hipStream_t st);
@@ -69,6 +71,10 @@ void launch_zero_u64(unsigned long long* d, int64_t n, hipStream_t st);
 // J (active cells and their periodic ghost copies) = acc * inv_scale
 void launch_j_from_fixed(const FieldView& J, const unsigned long long* acc, double inv_scale,
                          hipStream_t st);
+
+// J = the current of the accumulator after n filter passes; Bf is scratch
+void launch_filtered_current(const FieldView& J, const FieldView& Bf, const unsigned long long* acc,
+                             double inv_scale, int n, hipStream_t st);
 
 // ---- batched field launches over the boxes of an ensemble (fields.hip) ----
 struct FieldSeg {
@@ -111,15 +117,13 @@ ntt_status sort_batched(const SortSeg* segs, const int64_t* pbase, const int64_t
                         const int64_t* bbase, int64_t nblocks, int nseg, int64_t ptot,
                         int64_t ktot, uint32_t live, void* ws, hipStream_t st);
 
+// accumulators cleared by one launch
 struct FlatSeg {
-  void*       dst;
-  const void* src;
-  int64_t     n;      // elements
-  int64_t     blk0;
+  unsigned long long* dst;
+  int64_t             n;  // elements
+  int64_t             blk0;
 };
-enum { FLAT_ZERO_U64 = 0, FLAT_COPY_F32 = 1 };
 int64_t flat_seg_blocks(int64_t n);
-void    launch_flat_batched(int op, const FlatSeg* segs, int nseg, int64_t nblocks,
-                            hipStream_t st);
+void    launch_zero_batched(const FlatSeg* segs, int nseg, int64_t nblocks, hipStream_t st);
 
 }  // namespace ntt

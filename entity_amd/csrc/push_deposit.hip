@@ -63,14 +63,21 @@ template <> struct Win<2> {
 
 namespace {
 
-// Workgroup size and occupancy target of the fused kernel.  The LDS windows
-// (67.8 KB in 3D) admit two workgroups per CU; with 512 threads and at most
-// 128 VGPRs two workgroups give 4 waves per SIMD.
+// Workgroup size and occupancy target of the fused kernel.  The 3D LDS windows
+// (67.8 KB) admit two workgroups per CU; with 512 threads and at most 128 VGPRs
+// two workgroups give 4 waves per SIMD.  The 2D windows take 25 KB, so the
+// registers decide: held to 64 (a few spills) four workgroups give 8 waves per
+// SIMD.  Batched over 24 boxes of 64^2 to 128^2 cells: 171 us at order 2 and
+// 103 us at order 1, against 191 (98 registers, 4 waves) and 108 us (70, 6
+// waves) when only 4 waves are asked for.
 #ifndef NTT_PD_THREADS
 #define NTT_PD_THREADS 512
 #endif
 #ifndef NTT_PD_WAVES_PER_EU
 #define NTT_PD_WAVES_PER_EU 4
+#endif
+#ifndef NTT_PD_WAVES_PER_EU_2D
+#define NTT_PD_WAVES_PER_EU_2D 8
 #endif
 constexpr int kThreads = NTT_PD_THREADS;
 constexpr int kWaves   = kThreads / 64;
@@ -783,9 +790,8 @@ __device__ __forceinline__ int64_t tile_chunk(const FusedArgs& a) {
 // most of a small box's species on part of the GPU each: four species of 1.0e6
 // particles on 256 x 256 cells (order 1) take 85 us against 4 x 29 us.
 // The arguments are read in place, with an index uniform over the workgroup
-// (scalar loads from the kernel arguments): 70 registers at order 1, against 85
-// when a single species' arguments are a plain argument, hence six wavefronts
-// per SIMD instead of four.
+// (scalar loads from the kernel arguments): without a limit 70 registers at
+// order 1, against 85 when a single species' arguments are a plain argument.
 constexpr int kMergedSpecies = 8;
 struct FusedSpecies {
   FusedArgs a[kMergedSpecies];
@@ -795,7 +801,7 @@ struct FusedSpecies {
 static_assert(sizeof(FusedSpecies) <= 4096, "kernel argument block");
 
 template <int D, int O, int ALG>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NTT_PD_WAVES_PER_EU)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 2 ? NTT_PD_WAVES_PER_EU_2D : NTT_PD_WAVES_PER_EU)))
 void k_push_deposit(const FusedSpecies S) {
   const int64_t main = S.chunk0[S.n];
   const int64_t b    = blockIdx.x;
@@ -818,7 +824,7 @@ void k_push_deposit(const FusedSpecies S) {
 // The same over the boxes of an ensemble: entry e owns the global chunks
 // [chunk0[e], chunk0[e + 1]).
 template <int D, int O, int ALG>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NTT_PD_WAVES_PER_EU)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 2 ? NTT_PD_WAVES_PER_EU_2D : NTT_PD_WAVES_PER_EU)))
 void k_push_deposit_batched(const FusedArgs* __restrict__ table,
                             const int64_t* __restrict__ chunk0, int nent, int64_t nchunks) {
   const int64_t g = xcd_chunk(blockIdx.x, nchunks);

@@ -792,7 +792,10 @@ __device__ __forceinline__ int64_t tile_chunk(const FusedArgs& a) {
 // The arguments are read in place, with an index uniform over the workgroup
 // (scalar loads from the kernel arguments): without a limit 70 registers at
 // order 1, against 85 when a single species' arguments are a plain argument.
-constexpr int kMergedSpecies = 8;
+// Four species to a launch: the argument block of eight (3.6 KB) takes the host
+// longer to hand over, 3 to 4 us of a lone step of a 48 x 40 box (65 us against
+// 69), and boxes of more species fill the GPU with four.
+constexpr int kMergedSpecies = 4;
 struct FusedSpecies {
   FusedArgs a[kMergedSpecies];
   int64_t   chunk0[kMergedSpecies + 1];

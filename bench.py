@@ -517,6 +517,8 @@ def gr_run(N, a, *, ppc=8, rmax=50.0, theta=0.1, seed=4242, clear_interval=100, 
 
 # FP64 flop per particle-step of the GR push on the batched workload, from the
 # SQ_INSTS_VALU_{FMA,MUL,ADD,TRANS}_F64 counters (FMA counted twice)
+# of the kernel that divides per metric scalar; today's kernel executes fewer, so
+# rates from this count say how fast that work is done, not the issue rate
 GR_FP64_FLOP_PER_PARTICLE = 3506.0
 FP64_VECTOR_PEAK_TFLOPS = 78.6
 

@@ -269,8 +269,9 @@ __device__ __forceinline__ float out_of_plane(const KSMetric<RR, KIND>& M, RR x1
     double       v[3];
     m.to_cntrv(u, v);
     const double en = 1.0 + u1 * v[0] + u2 * v[1] + u3 * v[2];
-    // alpha / sqrt(en) with alpha^2 = Sigma / P
-    const double inv_energy = rsq64(en * m.P * m.iS);
+    // alpha / sqrt(en) with alpha^2 = Sigma / P (rsq64's steps turn an infinity
+    // into NaN)
+    const double inv_energy = isinf(en) ? 0.0 : rsq64(en * m.P * m.iS);
     return static_cast<float>(((isnan(v[2]) || isinf(v[2])) ? 0.0 : v[2]) * inv_energy);
   } else {
     MPt<RR> m;

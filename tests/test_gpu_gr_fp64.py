@@ -57,3 +57,35 @@ def test_gr_deposit_rows(hip, oracle, kind, n, npart):
     ref = np.zeros((3, n[1] + 2 * G, n[0] + 2 * G))
     assert oracle.gr_deposit(prm, h, ref, charge=-1.0, dt=float(np.float32(0.37))) == 0
     step._close(J.cpu().numpy(), ref, "J", rtol=4e-6)
+
+
+@pytest.mark.parametrize("kind", ["kerr_schild", "qkerr_schild", "kerr_schild_0"])
+@pytest.mark.parametrize("precision", [32, 64])
+def test_gr_deposit_infinite_momentum(hip, oracle, kind, precision):
+    """An infinite u_theta makes no out-of-plane current (the energy is infinite
+    and v^phi finite): J stays finite.  A NaN shows where its particle is."""
+    import torch
+
+    import test_gpu_gr_step as step
+    from entity_amd.containers import Particles
+    from entity_amd.kernels import device_errors, gr
+    n = (70, 30)
+    prm, met, shape = step._setup(oracle, kind, n, a=0.9 if kind != "kerr_schild_0" else 0.0)
+    h = step._gr_particles(np.random.default_rng(5), n, 600)
+    h["tag"][:] = 1
+    h["ux2"][3], h["ux2"][77], h["ux1"][300] = np.inf, -np.inf, np.nan
+    sp = Particles(2, 600, device="cuda", with_phi=True)
+    step._load(sp, h)
+    J = torch.zeros(shape.tensor_shape(3), device="cuda")
+    gr.DepositCurrents_kernel(J, shape, sp, met, -1.0, 0.37, precision)()
+    torch.cuda.synchronize()
+    assert device_errors() == 0
+    ref = np.zeros((3, n[1] + 2 * G, n[0] + 2 * G))
+    assert oracle.gr_deposit(prm, h, ref, charge=-1.0, dt=float(np.float32(0.37))) == 0
+    nan = np.isnan(ref)
+    assert 0 < nan.sum() <= 9
+    got = J.cpu().numpy()
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    ok = ~nan
+    # tolerances of test_gpu_gr_step.test_gr_deposit
+    step._close(got[ok], ref[ok], "J", rtol=4e-6 if precision == 64 else 2e-5)

@@ -447,10 +447,12 @@ void k_deposit(DepositArgs a) {
   if (live)
 #pragma unroll
     for (int d = 0; d < D; ++d) deposit_extent<O>(q.i[d], q.x[d], q.ip[d], q.xp[d], lo[d], hi[d]);
-  // the window holds offsets in [0, 1], moves of at most one cell and
-  // coefficients whose bound is a normal number with room for the scale
+  // the window holds offsets in [0, 1], moves of at most one cell, velocities
+  // that are numbers and coefficients whose bound is a normal number with room
+  // for the scale
   const float mag  = fabsf(q.coeff) * fmaxf(a.inv_dt, ONE);
-  bool        want = live && (mag == ZERO || (mag > 1.0e-28f && mag < 3.0e38f));
+  bool        want = live && fabsf(q.vz) <= TWO &&
+              (mag == ZERO || (mag > 1.0e-28f && mag < 3.0e38f));
   if (want)
 #pragma unroll
     for (int d = 0; d < D; ++d)

@@ -1,0 +1,71 @@
+"""What ntt_deposit_currents keeps of each contribution: momenta that are not
+finite."""
+import numpy as np
+import pytest
+import torch
+
+from _helpers import G, field_array
+
+pytestmark = pytest.mark.gpu
+
+DT = float(np.float32(0.35))
+
+
+def _deposit(p, dim, n, order):
+    from entity_amd.containers import GridShape, Particles
+    from entity_amd.kernels import DepositCurrents_kernel, Minkowski, device_errors
+    shape = GridShape(dim, n)
+    J = torch.zeros(shape.tensor_shape(3), device="cuda")
+    prt = Particles(dim, len(p["tag"])).load(**p)
+    DepositCurrents_kernel(J, shape, prt, Minkowski(dim), -1.0, DT, order)()
+    torch.cuda.synchronize()
+    assert device_errors() == 0
+    return J.cpu().numpy().astype(np.float64)
+
+
+def _oracle(oracle, p, dim, n, order, prec):
+    """The oracle's J, in FP64 with the single-precision builds' constant
+    0.333333 for a third where the scheme uses it."""
+    J = field_array(dim, n, 3, dtype=np.float32 if prec == "f32" else np.float64)
+    assert oracle.deposit(p, J, dim=dim, charge=-1.0, dt=DT, order=order, prec=prec) == 0
+    J = J.astype(np.float64)
+    if prec == "f64" and order > 0:
+        J[0 if dim == 3 else 2:] *= 3 * float(np.float32(0.333333))
+    return J
+
+
+def _tile_particles(dim, npart, seed, umax):
+    """Particles of one 8 x 4 x 4 tile, moved by less than half a cell."""
+    rng = np.random.default_rng(seed)
+    p = {}
+    for d in range(dim):
+        c = 8 + rng.integers(0, (8, 4, 4)[d], npart)
+        x = rng.random(npart).astype(np.float32) * np.float32(0.999)
+        y = x + rng.uniform(-0.45, 0.45, npart).astype(np.float32)
+        step = (y >= 1).astype(np.int32) - (y < 0).astype(np.int32)
+        p[f"i{d+1}"] = (c + step).astype(np.int32)
+        p[f"dx{d+1}"] = np.clip(y - step, 0, 1).astype(np.float32)
+        p[f"i{d+1}_prev"], p[f"dx{d+1}_prev"] = c.astype(np.int32), x
+    for d in range(3):
+        p[f"ux{d+1}"] = (umax * rng.standard_normal(npart)).astype(np.float32)
+    p["weight"] = np.ones(npart, np.float32)
+    p["tag"] = np.ones(npart, np.int16)
+    return p
+
+
+@pytest.mark.parametrize("order", [0, 1, 2])
+def test_nonfinite_momenta_2d(hip, oracle, order):
+    """A momentum that is not a number shows in the out-of-plane current of
+    exactly the cells its particle touches; an infinite one along the plane
+    makes none."""
+    n = (26, 18)
+    p = _tile_particles(2, 400, 11 + order, 0.5)
+    p["ux1"][17], p["ux2"][200], p["ux3"][399] = np.nan, np.inf, np.nan
+    got = _deposit(p, 2, n, order)
+    ref = _oracle(oracle, p, 2, n, order, "f64")
+    nan = np.isnan(ref)
+    assert nan[2].any() and not nan[:2].any()
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    # 400 contributions of at most 1/dt, a few roundings each
+    tol = 16 * 2.0 ** -24 / DT * 400
+    assert np.abs(got - ref)[~nan].max() <= tol

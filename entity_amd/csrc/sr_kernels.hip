@@ -1,8 +1,8 @@
 // sr_kernels.hip -- kernel-level SR pusher and current deposit over an
 // arbitrary (unsorted) particle range, reading E/B from HBM and accumulating J
 // at the reference's ghost-extended indices: per workgroup in an LDS window of
-// fixed point over the particles that are spatially close (then one FP32
-// atomic per touched entry), the others with FP32 atomics straight into J.
+// doubles over the particles that are spatially close (then one FP32 atomic
+// per touched entry), the others with FP32 atomics straight into J.
 //
 // These are the drop-ins for kernel::sr::Pusher_kernel and
 // kernel::DepositCurrents_kernel; the fused, tile-windowed push+deposit of
@@ -140,38 +140,36 @@ struct DepositArgs {
 };
 
 // Deposit of kDepThreads consecutive particles by one workgroup into an LDS
-// window of 64-bit fixed point, which is then added to J with one FP32 atomic
-// per non-zero entry.
+// window of doubles, which is then added to J with one FP32 atomic per non-zero
+// entry.
 //
 // The window is placed over the workgroup's particles, or, where they do not
 // fit one (a tile at the periodic boundary, whose wrapped particles deposit on
 // the far side of the array; a workgroup that straddles rows of tiles), over
 // those near the sample that most of the wavefronts' first particles are near.
-// The particles it leaves out, and all of them where it would take fewer than
-// kDepMin (its clearing and flush would cost more), are added to J directly.
+// The particles it leaves out, and all of them where such a window would take
+// fewer than kDepMin (its clearing and flush would cost more), are added to J
+// directly.
 //
-// Fixed point: the unit is a power of two chosen per workgroup so that the
-// largest contribution its heaviest particle can make, |charge weight| max(1/dt,
-// 1), stays below 2^30 units; particles more than 16 times lighter are added
-// directly.  A unit is then at most 2^-26 of the bound of any particle in the
-// window, below the 2^-25 that the single-precision shapes of the particle
-// already round to, and the sum of a cell is exact.  Against a window of
-// doubles the 3D order-2 kernel takes 0.82 instead of 1.04 ms per 1.7e7
-// particles (ds_add_u64 against ds_add_f64).
+// Every single-precision contribution of a particle in the window enters its
+// sum as it is, whatever the other particles' weights; the sum is rounded once.
+// (Sums of 32-bit fixed point in units of the heaviest particle's contribution,
+// ds_add_u64 for ds_add_f64, took 0.86 instead of 1.04 ms at the size below, but
+// lost what is small beside that particle: an error of 2.6e-4 in the J3 of a
+// plasma of |u| = 1e-4, against 3e-8 here.)
 //
 // In 3D (orders 1, 2) the accepted particles are reordered through an LDS
 // list, as in the step's deposit (push_deposit.hip): particles whose stencil
 // keeps its cells first (54 slots without per-slot branches at order 2), the
 // others by the direction they shift along, each rank-major by bank class.
 //
-// Measured on 128 x 128 x 64 cells, 1.7e7 particles in tile order, order 2:
-// 0.96 ms, of which loading and the box take 0.19 ms (4.7 TB/s of the
-// particles' 54 B), the list 0.27 ms, the stencils' arithmetic 0.3 ms, their LDS
-// atomics and the particles added directly the rest.  A window that is given
-// up, with every particle added by its own lane's FP32 atomics, where a
-// workgroup's box does not fit took 9.5 ms (the tiles at the periodic
-// boundary).  350 x 250 cells, order 1, 1.4e6 particles: 33 us (55 before).
-// In no order: 20 ms against 48 ms for one lane per particle.
+// Measured on 128 x 128 x 64 cells, 1.7e7 particles, order 2: 1.04 ms in tile
+// order and 1.27 ms four steps after it was made, with equal weights or weights
+// over four decades alike.  Giving the window up where a workgroup's box does not
+// fit it, every particle added by its own lane's FP32 atomics, took 9.3 and
+// 10.0 ms (the tiles at the periodic boundary).  In no order: 20 ms against 48.
+// 512 x 512 cells, 4.2e6 particles, order 1: 75 and 83 us, against 135 and 205.
+// kDepMin from 8 to 256: within 1% at 128 x 128 x 64 and 350 x 250 cells.
 constexpr int kDepThreads = 512;
 constexpr int kDepMin     = 64;
 
@@ -180,26 +178,22 @@ template <int D> struct DepWin;
 template <> struct DepWin<2> { static constexpr int W[3] = { 64, 16, 1 }; };
 template <> struct DepWin<3> { static constexpr int W[3] = { 14, 10, 10 }; };
 
-// window sink: values in units, below 2^31 (the 32-bit truncation, sign-extended)
+// window sink
 template <int D>
-struct LdsJw {
+struct LdsJd {
   static constexpr int W1 = DepWin<D>::W[0], W2 = DepWin<D>::W[1], WC = W1 * W2 * DepWin<D>::W[2];
-  unsigned long long* w;
-  int                 o1, o2, o3;
-  int                 base = 0;
+  double* w;
+  int     o1, o2, o3;
+  int     base = 0;
   __device__ __forceinline__ int index(int i, int j, int k) const {
     return (i - o1) + W1 * ((j - o2) + W2 * (k - o3));
   }
-  __device__ __forceinline__ void put(int at, float v) {
-    atomicAdd(w + at, static_cast<unsigned long long>(
-                        static_cast<long long>(static_cast<int32_t>(v))));
-  }
   __device__ __forceinline__ void set_origin(int i, int j, int k) { base = index(i, j, k); }
   __device__ __forceinline__ void add_rel(int a, int b, int g, int c, float v) {
-    put(c * WC + base + a + W1 * (b + W2 * g), v);
+    atomicAdd(w + c * WC + base + a + W1 * (b + W2 * g), static_cast<double>(v));
   }
   __device__ __forceinline__ void add(int i, int j, int k, int c, float v) {
-    put(c * WC + index(i, j, k), v);
+    atomicAdd(w + c * WC + index(i, j, k), static_cast<double>(v));
   }
 };
 
@@ -345,9 +339,9 @@ static_assert(kDepGroups == 64, "one wavefront scans the groups");
 // window through the list.  The caller has cleared the window, ctr and gsz and
 // passed a barrier.
 template <int O>
-__device__ __forceinline__ void deposit_listed(LdsJw<3>& jw, const int* org, int G, bool live,
-                                               const DepParticle<3>& q, float scale,
-                                               float inv_dt, DepListed* list, uint32_t (*ctr)[32],
+__device__ __forceinline__ void deposit_listed(LdsJd<3>& jw, const int* org, int G, bool live,
+                                               const DepParticle<3>& q, float inv_dt,
+                                               DepListed* list, uint32_t (*ctr)[32],
                                                uint32_t* gsz, uint32_t* gpos, uint32_t* counts) {
   const int tid = threadIdx.x, lane = tid & 63;
   uint32_t  cells = 0u;
@@ -392,7 +386,7 @@ __device__ __forceinline__ void deposit_listed(LdsJw<3>& jw, const int* org, int
     e.a = make_uint4(cells, __float_as_uint(q.x[0]), __float_as_uint(q.x[1]),
                      __float_as_uint(q.x[2]));
     e.b = make_uint4(__float_as_uint(q.xp[0]), __float_as_uint(q.xp[1]),
-                     __float_as_uint(q.xp[2]), __float_as_uint(q.coeff * scale));
+                     __float_as_uint(q.xp[2]), __float_as_uint(q.coeff));
     list[atomicAdd(&gpos[grp], 1u)] = e;
   }
   __syncthreads();
@@ -418,13 +412,6 @@ __device__ __forceinline__ void deposit_listed(LdsJw<3>& jw, const int* org, int
   }
 }
 
-// The window's unit: 2^k units per unit of current, the largest power of two
-// that keeps contributions of up to `bound` below 2^30 units.
-__device__ __forceinline__ float window_scale(float bound) {
-  const int e = bound > ZERO ? static_cast<int>((__float_as_uint(bound) >> 23) & 255u) - 127 : 0;
-  return ldexpf(ONE, max(-100, min(29 - e, 125)));
-}
-
 template <int D, int O>
 __global__ __launch_bounds__(kDepThreads) __attribute__((amdgpu_waves_per_eu(D == 3 && O > 0 ? 6 : 4)))
 void k_deposit(DepositArgs a) {
@@ -432,8 +419,8 @@ void k_deposit(DepositArgs a) {
   constexpr int  W1 = DepWin<D>::W[0], W2 = DepWin<D>::W[1], W3 = DepWin<D>::W[2];
   constexpr int  WC = W1 * W2 * W3;
   constexpr int  kWaves = kDepThreads / 64;
-  __shared__ unsigned long long jw[3 * WC];
-  __shared__ int       red[2 * D + 2][kWaves];
+  __shared__ double    jw[3 * WC];
+  __shared__ int       red[2 * D + 1][kWaves];
   __shared__ int       smp[kWaves][4];  // a particle of each wavefront: stencil start, valid
   __shared__ int       best, taken;
   __shared__ DepListed list[LIST ? kDepThreads : 1];
@@ -447,21 +434,14 @@ void k_deposit(DepositArgs a) {
   if (live)
 #pragma unroll
     for (int d = 0; d < D; ++d) deposit_extent<O>(q.i[d], q.x[d], q.ip[d], q.xp[d], lo[d], hi[d]);
-  // the window holds offsets in [0, 1], moves of at most one cell, velocities
-  // that are numbers and coefficients whose bound is a normal number with room
-  // for the scale
-  const float mag  = fabsf(q.coeff) * fmaxf(a.inv_dt, ONE);
-  bool        want = live && fabsf(q.vz) <= TWO &&
-              (mag == ZERO || (mag > 1.0e-28f && mag < 3.0e38f));
-  if (want)
+  // a listed particle's move is held in two bits per direction
+  bool want = live;
+  if constexpr (LIST)
 #pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (abs(q.ip[d] - q.i[d]) > 1 || !(q.x[d] >= ZERO && q.x[d] <= ONE) ||
-          !(q.xp[d] >= ZERO && q.xp[d] <= ONE))
-        want = false;
-  // over the workgroup (uniform): the box of the particles in `bits`, the
-  // largest coefficient, and whether every live one is in
-  auto box = [&](bool in, int* l, int* h, float& cmax) -> bool {
+    for (int d = 0; d < D; ++d) want = want && abs(q.ip[d] - q.i[d]) <= 1;
+  // over the workgroup (uniform): the box of the particles that are `in`, and
+  // whether every live one is
+  auto box = [&](bool in, int* l, int* h) -> bool {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int bl = wave_reduce<false>(in ? lo[d] : INT_MAX);
@@ -471,12 +451,8 @@ void k_deposit(DepositArgs a) {
         red[2 * d + 1][wv] = bh;
       }
     }
-    const int  cm  = wave_reduce<true>(in ? __float_as_int(mag) : 0);
     const bool all = __ballot(live && !in) == 0ull;
-    if (lane == 0) {
-      red[2 * D][wv]     = cm;
-      red[2 * D + 1][wv] = all;
-    }
+    if (lane == 0) red[2 * D][wv] = all;
     __syncthreads();
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -489,26 +465,22 @@ void k_deposit(DepositArgs a) {
       l[d] = __builtin_amdgcn_readfirstlane(bl);  // uniform: scalar registers
       h[d] = __builtin_amdgcn_readfirstlane(bh);
     }
-    int c = red[2 * D][0], every = red[2 * D + 1][0];
+    int every = red[2 * D][0];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) {
-      c = max(c, red[2 * D][w]);
-      every &= red[2 * D + 1][w];
-    }
-    cmax = __int_as_float(__builtin_amdgcn_readfirstlane(c));
+    for (int w = 1; w < kWaves; ++w) every &= red[2 * D][w];
     return __builtin_amdgcn_readfirstlane(every) != 0;
   };
   if (tid == 0) best = taken = 0;
-  for (int k = tid; k < 3 * WC; k += kDepThreads) jw[k] = 0ull;
+  for (int k = tid; k < 3 * WC; k += kDepThreads) jw[k] = 0.0;
   if constexpr (LIST)
     if (tid < 160 + kDepGroups) {
       if (tid < 160) ctr[tid >> 5][tid & 31] = 0u;
       else gsz[tid - 160] = 0u;
     }
-  int   org[3] = { 0, 0, 0 }, top[3] = { 0, 0, 0 };
-  float cmax;
-  bool  fits = box(want, org, top, cmax);
+  int  org[3] = { 0, 0, 0 }, top[3] = { 0, 0, 0 };
+  bool fits = box(want, org, top);
   const bool empty = org[0] > top[0];  // nothing for the window
+  fits = fits && !empty;
 #pragma unroll
   for (int d = 0; d < D; ++d)
     fits = fits && static_cast<int64_t>(top[d]) - org[d] < DepWin<D>::W[d];
@@ -532,7 +504,7 @@ void k_deposit(DepositArgs a) {
     }
     __syncthreads();
     const int ref = __builtin_amdgcn_readfirstlane(best) % kWaves;
-    box(want && near_sample(lo, ref), org, top, cmax);
+    box(want && near_sample(lo, ref), org, top);
     // a box wider than the window: from a quarter window below the sample
 #pragma unroll
     for (int d = 0; d < D; ++d)
@@ -541,7 +513,7 @@ void k_deposit(DepositArgs a) {
           max(org[d], smp[ref][d] - DepWin<D>::W[d] / 4));
   }
   // the particles the window takes
-  bool in = want && (mag * 16.0f >= cmax || mag == ZERO);
+  bool in = want;
 #pragma unroll
   for (int d = 0; d < D; ++d) in = in && lo[d] >= org[d] && hi[d] < org[d] + DepWin<D>::W[d];
   const uint64_t out = __ballot(live && !in);
@@ -550,7 +522,7 @@ void k_deposit(DepositArgs a) {
     if (lane == 0 && b != 0ull) atomicAdd(&taken, __popcll(b));
   }
   __syncthreads();
-  const bool window = __builtin_amdgcn_readfirstlane(taken) >= kDepMin;
+  const bool window = fits || __builtin_amdgcn_readfirstlane(taken) >= kDepMin;
   uint64_t   direct = window ? out : __ballot(live);
   if constexpr (LIST) {
 #pragma unroll 1
@@ -575,28 +547,22 @@ void k_deposit(DepositArgs a) {
     }
   }
   if (!window) return;
-  const float scale = window_scale(cmax);
-  LdsJw<D>    J{ jw, org[0] + G, org[1] + G, D == 3 ? org[2] + G : 0 };
-  if constexpr (LIST) {
-    deposit_listed<O>(J, org, G, in, q, scale, a.inv_dt, list, ctr, gsz, gpos, counts);
-  } else if (in) {
-    q.coeff *= scale;
-    deposit_one<D, O>(J, G, q, a.inv_dt);
-  }
+  LdsJd<D> J{ jw, org[0] + G, org[1] + G, D == 3 ? org[2] + G : 0 };
+  if constexpr (LIST) deposit_listed<O>(J, org, G, in, q, a.inv_dt, list, ctr, gsz, gpos, counts);
+  else if (in) deposit_one<D, O>(J, G, q, a.inv_dt);
   __syncthreads();
-  const double unit = 1.0 / static_cast<double>(scale);
-  const int    e1 = min(top[0] - org[0] + 1, W1), e2 = min(top[1] - org[1] + 1, W2);
-  const int    rows = (D == 3 ? min(top[2] - org[2] + 1, W3) : 1) * (W1 * W2);
+  const int e1 = min(top[0] - org[0] + 1, W1), e2 = min(top[1] - org[1] + 1, W2);
+  const int rows = (D == 3 ? min(top[2] - org[2] + 1, W3) : 1) * (W1 * W2);
   for (int e = tid; e < rows; e += kDepThreads) {
     const int z = e / (W1 * W2), t = e - z * (W1 * W2);
     const int y = t / W1, x = t - y * W1;
     if (x < e1 && y < e2) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        const long long v = static_cast<long long>(jw[c * WC + e]);
-        if (v != 0)
+        const double v = jw[c * WC + e];
+        if (v != 0.0)
           a.J.add(org[0] + G + x, org[1] + G + y, D == 3 ? org[2] + G + z : 0, c,
-                  static_cast<float>(static_cast<double>(v) * unit));
+                  static_cast<float>(v));
       }
     }
   }

@@ -1,5 +1,6 @@
-"""What ntt_deposit_currents keeps of each contribution: momenta that are not
-finite."""
+"""What ntt_deposit_currents keeps of each contribution: particles much lighter
+than their neighbours, a cold plasma's out-of-plane current, and momenta that
+are not finite."""
 import numpy as np
 import pytest
 import torch
@@ -51,6 +52,35 @@ def _tile_particles(dim, npart, seed, umax):
     p["weight"] = np.ones(npart, np.float32)
     p["tag"] = np.ones(npart, np.int16)
     return p
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("light", [1.0 / 15, 1e-4])
+def test_light_and_cold(hip, oracle, dim, order, light):
+    """Light particles share their workgroups with heavy ones, and the plasma is
+    cold (|u| of 1e-4).  Per component, over the cells that only light particles
+    reach and over the others, the error against 64 bits is at most twice that
+    of the same sums in FP32 throughout: a contribution takes the same few
+    roundings in both, and the window's sum fewer than the FP32 oracle's."""
+    n = (26, 18) if dim == 2 else (26, 18, 17)
+    p = _tile_particles(dim, 1500, 3 * order + dim, 1e-4)
+    p["weight"][p["i1_prev"] >= 11] = light
+    ref = _oracle(oracle, p, dim, n, order, "f64")
+    f32 = np.abs(_oracle(oracle, p, dim, n, order, "f32") - ref)
+    err = np.abs(_deposit(p, dim, n, order) - ref)
+    # magnitudes that meet in each entry
+    A = {True: np.zeros_like(ref), False: np.zeros_like(ref)}
+    for k in range(len(p["tag"])):
+        q = {name: v[k:k + 1] for name, v in p.items()}
+        A[bool(p["weight"][k] < 1)] += np.abs(_oracle(oracle, q, dim, n, order, "f64"))
+    for mask in ((A[False] == 0) & (A[True] > 0), A[False] > 0):
+        for c in range(3):
+            m = mask[c]
+            S = (A[True] + A[False])[c][m].sum()
+            assert m.sum() > 20
+            assert err[c][m].sum() <= 2 * f32[c][m].sum(), (c, err[c][m].sum() / S,
+                                                            f32[c][m].sum() / S)
 
 
 @pytest.mark.parametrize("order", [0, 1, 2])

@@ -156,7 +156,7 @@ struct DepositArgs {
 // (Sums of 32-bit fixed point in units of the heaviest particle's contribution,
 // ds_add_u64 for ds_add_f64, took 0.86 instead of 1.04 ms at the size below, but
 // lost what is small beside that particle: an error of 2.6e-4 in the J3 of a
-// plasma of |u| = 1e-4, against 3e-8 here.)
+// plasma of |u| = 1e-4, against 3e-8 with FP32 sums throughout.)
 //
 // In 3D (orders 1, 2) the accepted particles are reordered through an LDS
 // list, as in the step's deposit (push_deposit.hip): particles whose stencil
@@ -164,11 +164,11 @@ struct DepositArgs {
 // others by the direction they shift along, each rank-major by bank class.
 //
 // Measured on 128 x 128 x 64 cells, 1.7e7 particles, order 2: 1.04 ms in tile
-// order and 1.27 ms four steps after it was made, with equal weights or weights
+// order and 1.30 ms four steps after it was made, with equal weights or weights
 // over four decades alike.  Giving the window up where a workgroup's box does not
 // fit it, every particle added by its own lane's FP32 atomics, took 9.3 and
 // 10.0 ms (the tiles at the periodic boundary).  In no order: 20 ms against 48.
-// 512 x 512 cells, 4.2e6 particles, order 1: 75 and 83 us, against 135 and 205.
+// 512 x 512 cells, 4.2e6 particles, order 1: 74 and 83 us, against 135 and 205.
 // kDepMin from 8 to 256: within 1% at 128 x 128 x 64 and 350 x 250 cells.
 constexpr int kDepThreads = 512;
 constexpr int kDepMin     = 64;
@@ -271,46 +271,58 @@ __device__ __forceinline__ float lane_value(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// Weight of the order-O shape of a particle at distance t from a node, and
-// the sum of its weights on the nodes up to that one (shape_order<false, O>
-// by the node's distance).
-template <int O>
-__device__ __forceinline__ void node_weight(float t, float& w, float& cum) {
-  if constexpr (O == 1) {
-    w   = fmaxf(ONE - fabsf(t), ZERO);
-    cum = t <= ZERO ? w : ONE;
-  } else {
-    const float far = fmaxf(THREE_HALFS - fabsf(t), ZERO), up = fmaxf(HALF - t, ZERO);
-    w   = fabsf(t) <= HALF ? THREE_FOURTHS - t * t : HALF * (far * far);
-    cum = t <= -HALF ? w : ONE - HALF * (up * up);  // 1 - the next node's weight
-  }
+// entry s of v, s differing between the lanes (starting from zero, not v[0]: a
+// choice between two entries becomes one of addresses, and v goes to scratch)
+template <int M>
+__device__ __forceinline__ float entry(const float (&v)[M], int s) {
+  float r = ZERO;
+#pragma unroll
+  for (int k = 0; k < M; ++k) r = s == k ? v[k] : r;
+  return r;
 }
 
 // The 3D Esirkepov deposit (O = 1, 2) of one particle, the same for the whole
 // wavefront, straight into J: lane a + 4 b + 16 g takes stencil slot (a, b, g)
-// of the three components.  The slots' values are those of
-// deposit_esirkepov_3d up to rounding.
+// of the three components.  Shapes, longitudinal coefficients and products are
+// those of deposit_esirkepov_3d.
 template <int O>
 __device__ __forceinline__ void deposit_wave(const GlobalJ& J, int G, const DepParticle<3>& q,
                                              float inv_dt) {
-  const int lane = threadIdx.x & 63;
-  const int s[3] = { lane & 3, (lane >> 2) & 3, lane >> 4 };
-  int       m[3], n[3];
-  float     iS[3], fS[3], C[3];
-  bool      in = true;
+  constexpr int M = O + 2;
+  const int   lane = threadIdx.x & 63;
+  const int   s[3] = { lane & 3, (lane >> 2) & 3, lane >> 4 };
+  const float q3   = -(q.coeff * inv_dt) * THIRD;
+  int         m[3], n[3];
+  float       iS[3], fS[3], C[3];
+  bool        in = true;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    // first nodes of the shapes before and after, relative to their cells; the
-    // one further up starts at slot 1 (for_deposit)
-    const int a = (O == 2 && q.xp[d] < HALF) ? -1 : 0, b = (O == 2 && q.x[d] < HALF) ? -1 : 0;
-    const int ga = q.ip[d] + a, gb = q.i[d] + b;
-    m[d] = min(ga, gb);
-    n[d] = (ga == gb) ? O : O + 1;
+    int   a, b;
+    float Si[O + 1], Sf[O + 1], i[M], f[M], c[O + 1];
+    shape_order<false, O, true>(q.ip[d], q.xp[d], a, Si);
+    shape_order<false, O, true>(q.i[d], q.x[d], b, Sf);
+    // for_deposit, with selects: the shape that starts further up begins at slot 1
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      i[k] = f[k] = ZERO;
+      if (k <= O) {
+        i[k] = a > b ? ZERO : Si[k];
+        f[k] = b > a ? ZERO : Sf[k];
+      }
+      if (k > 0) {
+        i[k] = a > b ? Si[k - 1] : i[k];
+        f[k] = b > a ? Sf[k - 1] : f[k];
+      }
+    }
+    m[d] = min(a, b);
+    n[d] = (a == b) ? O : O + 1;
     in   = in && s[d] <= n[d];
-    float ci, cf;
-    node_weight<O>(static_cast<float>(a + s[d] - (ga > gb ? 1 : 0)) - q.xp[d], iS[d], ci);
-    node_weight<O>(static_cast<float>(b + s[d] - (gb > ga ? 1 : 0)) - q.x[d], fS[d], cf);
-    C[d] = -(q.coeff * inv_dt) * THIRD * (cf - ci);
+    c[0] = q3 * (f[0] - i[0]);
+#pragma unroll
+    for (int k = 1; k <= O; ++k) c[k] = fmaf(q3, f[k] - i[k], c[k - 1]);
+    iS[d] = entry(i, s[d]);
+    fS[d] = entry(f, s[d]);
+    C[d]  = entry(c, s[d]);
   }
   if (!in) return;
   GlobalJ w = J;

@@ -1,6 +1,6 @@
 """What ntt_deposit_currents keeps of each contribution: particles much lighter
-than their neighbours, a cold plasma's out-of-plane current, and momenta that
-are not finite."""
+than their neighbours, a cold plasma's out-of-plane current, particles next to
+a node that are added to J directly, and momenta that are not finite."""
 import numpy as np
 import pytest
 import torch
@@ -99,3 +99,36 @@ def test_nonfinite_momenta_2d(hip, oracle, order):
     # 400 contributions of at most 1/dt, a few roundings each
     tol = 16 * 2.0 ** -24 / DT * 400
     assert np.abs(got - ref)[~nan].max() <= tol
+
+
+@pytest.mark.parametrize("order", [1, 2])
+def test_direct_near_nodes_3d(hip, oracle, order):
+    """Particles too far apart for a window, moving along x, next to a node (order
+    1) or to the middle of their cell (order 2) along y and z, where one weight
+    is tiny: it keeps its relative accuracy, so every slot of J1 does.  The
+    longitudinal factor (a difference of shapes that move by 0.4 of a cell)
+    takes under 8 roundings of its value, each transverse product 3 (all of one
+    sign)."""
+    n = (60, 55, 50)
+    k = np.arange(30)
+    p = {}
+    for d in range(3):
+        c = ((7 * k, 11 * k, 13 * k)[d] % (n[d] - 8) + 4).astype(np.int32)
+        p[f"i{d+1}"], p[f"i{d+1}_prev"] = c, c.copy()
+    tiny = np.float32(10.0) ** np.linspace(-6.5, -3, 30).astype(np.float32)
+    at = np.float32(0.5 if order == 2 else 0.0)
+    p["dx1_prev"] = np.full(30, 0.55, np.float32)
+    p["dx1"] = np.full(30, 0.95, np.float32)
+    for d in (2, 3):
+        sign = -1 if order == 2 else 1
+        p[f"dx{d}_prev"] = (at + sign * tiny).astype(np.float32)
+        p[f"dx{d}"] = (at + sign * 3 * tiny).astype(np.float32)
+    for d in range(3):
+        p[f"ux{d+1}"] = np.zeros(30, np.float32)
+    p["weight"] = np.ones(30, np.float32)
+    p["tag"] = np.ones(30, np.int16)
+    got, ref = _deposit(p, 3, n, order)[0], _oracle(oracle, p, 3, n, order, "f64")[0]
+    m = np.abs(ref) > 1e-30
+    assert m.sum() >= 30 * 4
+    assert (np.abs(got - ref)[m] <= 16 * 2.0 ** -24 * np.abs(ref)[m]).all(), \
+        (np.abs(got - ref)[m] / np.abs(ref)[m]).max()

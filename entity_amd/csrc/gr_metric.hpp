@@ -290,9 +290,11 @@ struct KSMetric {
 // ---- FP64 points of the Kerr-Schild and quasi-spherical metrics ---------------
 // The metric's formulas regrouped around one reciprocal per point, with
 // reciprocals and reciprocal roots from the hardware estimate and two Newton
-// steps (about 1 ulp) in the place of IEEE divisions and roots.  A point a
-// fraction of a cell away from another takes its exp, sin and cos from that
-// one's by the addition theorems.
+// steps (at most 0.5 and 1.6 ulp) in the place of IEEE divisions and roots.  A
+// point a fraction of a cell away from another takes its exp, sin and cos from
+// that one's by the addition theorems, unless it is that much nearer to the
+// axis that the sine would lose digits.  Zero and infinity come out of the
+// Newton steps as NaN.
 __device__ __forceinline__ double rcp64(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = fma(r, fma(-x, r, 1.0), r);
@@ -405,7 +407,9 @@ struct FastPoint {
     const double dth = th - b.th;
     double       dchi = 0.0;
     if constexpr (KIND == NTT_METRIC_QKERR_SCHILD) dchi = (x1 - b1) * M.k.dchi;
-    if (fabs(dth) <= kNear && fabs(dchi) <= kNear) {
+    // up to a quarter of b's distance from the axis: sin stays within 4e-16 of
+    // itself (half of it: 6e-16; from 0.02 to 1e-5 rad the two terms cancel to 1e-12)
+    if (fabs(dth) <= fmin(kNear, 0.25 * b.s) && fabs(dchi) <= kNear) {
       double sd, cd;
       sin_cos_near(dth, &sd, &cd);
       s = fma(b.c, sd, b.s * cd);

@@ -31,6 +31,24 @@ def test_midpoints_near_and_far(hip, oracle, monkeypatch, metric, massless, n, d
     base._compare(got, ref, rtol=2e-6, xtol=2 * float(np.spacing(np.float32(max(n)))), inp=p)
 
 
+@pytest.mark.parametrize("metric", ["ks", "qks", "qks_h"])
+@pytest.mark.parametrize("massless", [False, True])
+@pytest.mark.parametrize("dt", [0.001, 0.02])
+def test_midpoints_next_to_the_axis(hip, oracle, monkeypatch, metric, massless, dt):
+    """A fine grid with an eighth of the particles in the cells next to the axis,
+    whose midpoints lie closer to it than a quarter of their own distance or
+    further: on both sides of that line (fields off, as in
+    test_gr_axis_massive_zero_fields)."""
+    n = (400, 300)
+    monkeypatch.setattr(base, "N", n)
+    em = np.zeros((6, n[1] + 2 * G, n[0] + 2 * G), np.float32)
+    p = base._particles(12, npart=1500, umax=0.3, near_axis=True)
+    got = base._run_gpu(hip, metric, p, em, em, massless=massless, order=1, precision=64, dt=dt)
+    ref = base._run_oracle(oracle, metric, p, em, em, massless=massless, order=1, prec="f64",
+                           dt=dt)
+    base._compare(got, ref, rtol=2e-6, xtol=2 * float(np.spacing(np.float32(max(n)))), inp=p)
+
+
 @pytest.mark.parametrize("kind", ["kerr_schild", "qkerr_schild", "kerr_schild_0"])
 @pytest.mark.parametrize("n,npart", [((150, 24), 9001), ((70, 30), 5000), ((131, 9), 1)])
 def test_gr_deposit_rows(hip, oracle, kind, n, npart):

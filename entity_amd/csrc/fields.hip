@@ -528,10 +528,18 @@ __global__ __launch_bounds__(FTX* FTY) void k_filter_periodic_3d(FieldView Dst, 
 }
 
 // A workgroup marches nk planes.  16 where that gives four workgroups a CU;
-// smaller grids halve it until it does, since a march is a chain of plane loads
-// (70 x 184 x 38 cells: 20.5 us with 16 planes, 10.7 with 4; 230 x 159 x 44:
-// 21.4 with 16, 15.9 with 8, 18.7 with 4; 250 x 156 x 131: 36 with 16, 40 with 8
-// and the planes around each march read again).
+// smaller grids halve it until it does, since a march is a chain of plane loads,
+// while a longer one reads fewer planes twice.  us per pass (* what the rule
+// takes, within 2% of the best on each):
+//   cells              2        4        8       16
+//   100 x 84 x 58     9.3 *    9.4     12.2     18.3
+//   70 x 184 x 38    10.7 *   11.1     12.8     20.3
+//   128 x 128 x 64   11.9     11.4 *   13.1     18.7
+//   230 x 159 x 44   18.7     15.9 *   17.3     21.4
+//   32 x 200 x 200   20.9     19.3     19.7 *   24.2
+//   300 x 300 x 20   21.1     18.1     16.9 *   22.0
+//   250 x 156 x 131  48.0     42.5     39.7     35.9 *
+//   247 x 207 x 227   113       95       93       94 *
 constexpr int64_t kFilterBlocks = 1024;
 template <bool GHOSTS>
 void launch_filter_3d(const FieldView& dst, const FieldView& src, hipStream_t st) {

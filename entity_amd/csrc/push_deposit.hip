@@ -69,7 +69,14 @@ namespace {
 // registers decide: held to 64 (a few spills) four workgroups give 8 waves per
 // SIMD.  Batched over 24 boxes of 64^2 to 128^2 cells: 171 us at order 2 and
 // 103 us at order 1, against 191 (98 registers, 4 waves) and 108 us (70, 6
-// waves) when only 4 waves are asked for.
+// waves) when only 4 waves are asked for.  Single boxes, order 0 / 1 / 2, us
+// per step of all species, 8 waves asked for (4):
+//   512^2, 2 species    Boris 190 / 191 / 260 (206 / 204 / 285), Vay 192 / 190 /
+//                       254 (206 / 209 / 287), photons 165 (169)
+//   344 x 248, 2        Boris 58 / 53 / 78 (60 / 57 / 91), Vay 59 / 55 / 79
+//                       (61 / 58 / 93), photons 32 (34)
+//   64^2, 2             Boris 19 / 20 / 23 (18 / 18 / 22), photons 14 (13): too
+//                       few workgroups for the occupancy to matter
 #ifndef NTT_PD_THREADS
 #define NTT_PD_THREADS 512
 #endif

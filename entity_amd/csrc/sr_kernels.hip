@@ -80,12 +80,12 @@ __device__ __forceinline__ bool gather_in_array(const PushArgs& a, const PState&
 }
 
 // One particle per thread.  Bound by the gather's loads through the caches
-// (162 per particle in 3D at order 2): issued a component at a time
-// (GlobalEMAhead), 1.7e7 particles in tile order on 128 x 128 x 64 cells take
-// 0.81 ms (1.03 ms on average between re-sorts 4 steps apart; 1.56 ms with the
-// compiler's own order, which waits for every row), 512 x 512 cells at order 2
-// 81 us (115).  139 registers, three wavefronts per SIMD: held to 128 or 96
-// registers it spills and takes 0.94 and 1.17 ms.
+// (162 values per particle in 3D at order 2, a stencil row of 3 in one load):
+// issued a component at a time (GlobalEMAhead), 1.7e7 particles in tile order on
+// 128 x 128 x 64 cells take 0.81 ms (1.03 ms on average between re-sorts 4 steps
+// apart; 1.56 ms with the compiler's own order, which waits for every row), 512
+// x 512 cells at order 2 81 us (115).  139 registers, three wavefronts per SIMD:
+// held to 128 or 96 registers it spills and takes 0.94 and 1.17 ms.
 template <int D, int O, int ALG>
 __global__ __launch_bounds__(kBlock) void k_sr_push(PushArgs a) {
   const int64_t  base = static_cast<int64_t>(blockIdx.x) * kBlock;

@@ -1,7 +1,7 @@
 """ntt_deposit_currents against the FP64 oracle where its LDS window can go
 wrong: particle counts around a workgroup's, particles in tile order, across
 the periodic boundary, across rows of tiles, in no order, and weights over many
-decades (the window's fixed point is chosen per workgroup)."""
+decades."""
 import numpy as np
 import pytest
 import torch

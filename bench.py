@@ -515,11 +515,12 @@ def gr_run(N, a, *, ppc=8, rmax=50.0, theta=0.1, seed=4242, clear_interval=100, 
     return run
 
 
-# FP64 flop per particle-step of the GR push on the batched workload, from the
-# SQ_INSTS_VALU_{FMA,MUL,ADD,TRANS}_F64 counters (FMA counted twice)
-# of the kernel that divides per metric scalar; today's kernel executes fewer, so
-# rates from this count say how fast that work is done, not the issue rate
-GR_FP64_FLOP_PER_PARTICLE = 3506.0
+# FP64 flop per particle-step (SQ_INSTS_VALU_{FMA,MUL,ADD,TRANS}_F64, FMA counted
+# twice) and VALU instructions per 64 particles of the GR push on the batched
+# workload
+GR_COUNTERS_PROFILE = "k_gr_push_batched_qks_16x768x768_counters.md"
+GR_FP64_FLOP_PER_PARTICLE = 1579.0
+GR_VALU_PER_64 = 1571.0
 FP64_VECTOR_PEAK_TFLOPS = 78.6
 
 
@@ -570,7 +571,10 @@ def gr_leg(args):
                          "peak": FP64_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": tflops / FP64_VECTOR_PEAK_TFLOPS,
                          "flop_per_particle_step": GR_FP64_FLOP_PER_PARTICLE,
-                         "flop_source": "profiles/k_gr_push_qks_768x768_counters.md"}}
+                         "flop_source": f"profiles/{GR_COUNTERS_PROFILE}",
+                         "valu_frac": rate / 64 * GR_VALU_PER_64 / (MI355X_CUS * MI355X_CLOCK_HZ),
+                         "valu_source": f"profiles/{GR_COUNTERS_PROFILE} (SQ_INSTS_VALU per 64 "
+                                        "particles) x the rate / (256 CUs x 2.4 GHz)"}}
 
 
 def gr_full_leg(args):
@@ -812,9 +816,9 @@ def beams2d_leg(args, tuned=None):
     ms, nl = C.c_double(0), C.c_int64(0)
     _abi.check(lib.ntt_profile_read(C.byref(ms), C.byref(nl), 1), "ntt_profile_read")
     npart = 4 * n[0] * n[1] * ppc
-    per = n[0] * n[1] * ppc
-    avg = ms.value / max(nl.value, 1)
-    achieved = (per * 78 + n[0] * n[1] * 36) / (avg * 1e-3) / 1e9
+    # one launch a step holds the four species: particles, and E/B and J once
+    avg = ms.value / nsteps
+    achieved = (npart * 78 + n[0] * n[1] * 36) / (avg * 1e-3) / 1e9
     out = {"workload": "2D periodic 256x256, e-/e+ beams u_x +-0.57735 over theta 0.1, "
                        "4 species x 16 ppc (4,194,304 particles), order 1, Boris, 1 filter pass, "
                        "100 steps",
@@ -822,7 +826,8 @@ def beams2d_leg(args, tuned=None):
            "particles": npart, "steps": nsteps, "value": npart * nsteps / el,
            "unit": "particle-steps/s", "ms_per_step": 1e3 * el / nsteps,
            "cell_updates_per_s": n[0] * n[1] * nsteps / el,
-           "fused_kernel": {"avg_launch_ms": avg, "achieved_gbs": achieved,
+           "fused_kernel": {"avg_launch_ms": avg, "species_per_launch": 4,
+                            "achieved_gbs": achieved,
                             "frac": achieved / HBM_PEAK_GBS}}
     if args.cpu_baseline:
         out["cpu_baseline"] = beams2d_cpu_baseline(eng, n, ppc, drifts)
@@ -951,7 +956,7 @@ def main():
             "kernel": (SPLIT_KERNELS + " (push with E/B from LDS, then Esirkepov deposit into "
                        "LDS windows; one species per pair, timed together)")
                       if dim == 3 and args.order in (1, 2) else
-                      "k_push_deposit (fused push + Esirkepov deposit, one species per launch)",
+                      "k_push_deposit (fused push + Esirkepov deposit, time per species)",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",

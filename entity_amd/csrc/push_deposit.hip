@@ -801,7 +801,8 @@ __device__ __forceinline__ int64_t tile_chunk(const FusedArgs& a) {
 // order 1, against 85 when a single species' arguments are a plain argument.
 // Four species to a launch: the argument block of eight (3.6 KB) takes the host
 // longer to hand over, 3 to 4 us of a lone step of a 48 x 40 box (65 us against
-// 69), and boxes of more species fill the GPU with four.
+// 69; 12 us of a new box's first step, 125 against 137), and boxes of more
+// species fill the GPU with four.
 constexpr int kMergedSpecies = 4;
 struct FusedSpecies {
   FusedArgs a[kMergedSpecies];
